@@ -491,6 +491,138 @@ struct PolF32 {
     }
 };
 
+// ------------------------------------------------- fp32 products in bf16 parts
+
+// An fp32 value is the sum of three bf16 values h + m + l (each the nearest
+// bf16 to what is left, so |m| <= 2^-9 |x| and |l| <= 2^-18 |x|; 24 bits in
+// all). A product of two such sums is six bf16 products, exact in fp32 and
+// accumulated there; the three left out (m l, l m, l l) are below 2^-26 of
+// |x y|, a quarter of an fp32 rounding. v_mfma_f32_16x16x32_bf16 runs at 16
+// times the rate of v_mfma_f32_16x16x4_f32, so the six take 3/8 of its time,
+// and a 16x16 tile's sums over 64 elements are rounded 12 times instead of
+// 16. Operands hold 8 consecutive elements per lane, in PolBF16's layout.
+struct Split3 {
+    bf16x8 h, m, l;
+};
+
+//
+// The parts of an infinity, or of a value that rounds to one in bf16, are NaN
+// (inf - inf), as are those of its neighbour in a pair; kernels that use them
+// check their results and, on any that is not finite, run the work-group again
+// with v_mfma_f32_16x16x4_f32.
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
+// One part of a pair: the nearest bf16s, packed, and what is left of each
+// element (exact). 5 plain VALU instructions. One v_dot2_f32_bf16 against (-1,
+// 0) or (0, -1) would unpack and subtract at once, but it runs on the matrix
+// unit, and next to MFMAs (also other waves') takes 15-20 cycles where the two
+// instructions it replaces take 8 and hide behind them.
+__device__ __forceinline__ uint32_t part_of(float &x, float &y) {
+    uint32_t h = __builtin_bit_cast(uint32_t, bf16x2{(__bf16)x, (__bf16)y});
+    asm("" : "+v"(h));  // else each element is converted a second time on its own
+    x -= __uint_as_float(h << 16);
+    y -= __uint_as_float(h & 0xffff0000u);
+    return h;
+}
+
+__device__ __forceinline__ Split3 split3(const f32x4 &a, const f32x4 &b) {
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    u32x4 h, m, l;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float x = i < 2 ? a[2 * i] : b[2 * i - 4], y = i < 2 ? a[2 * i + 1] : b[2 * i - 3];
+        h[i] = part_of(x, y);
+        m[i] = part_of(x, y);
+        l[i] = __builtin_bit_cast(uint32_t, bf16x2{(__bf16)x, (__bf16)y});
+    }
+    return Split3{__builtin_bit_cast(bf16x8, h), __builtin_bit_cast(bf16x8, m), __builtin_bit_cast(bf16x8, l)};
+}
+
+// c + A B over NC k-steps: the smallest products first, so that only the last
+// NC are rounded at the size of the result.
+template <int NC>
+__device__ __forceinline__ f32x4 mma_split(const Split3 (&a)[NC], const Split3 (&b)[NC], f32x4 c) {
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[k].l, b[k].h, c, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[k].h, b[k].l, c, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[k].m, b[k].m, c, 0, 0, 0);
+    }
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[k].m, b[k].h, c, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[k].h, b[k].m, c, 0, 0, 0);
+    }
+#pragma unroll
+    for (int k = 0; k < NC; ++k) c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[k].h, b[k].h, c, 0, 0, 0);
+    return c;
+}
+
+// c[t][u] += A_t B_u for T x U tiles, product by product over all the tiles, so
+// that consecutive matrix instructions are independent.
+template <int NC, int T, int U>
+__device__ __forceinline__ void mma_split_tiles(f32x4 (&c)[T][U], const Split3 (&a)[T][NC], const Split3 (&b)[U][NC]) {
+    auto each = [&](auto mma) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < NC; ++k) {
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+#pragma unroll
+                for (int u = 0; u < U; ++u) c[t][u] = mma(a[t][k], b[u][k], c[t][u]);
+            }
+        }
+    };
+    each([](const Split3 &x, const Split3 &y, f32x4 v) { return PolBF16<64>::mma(x.l, y.h, v); });
+    each([](const Split3 &x, const Split3 &y, f32x4 v) { return PolBF16<64>::mma(x.h, y.l, v); });
+    each([](const Split3 &x, const Split3 &y, f32x4 v) { return PolBF16<64>::mma(x.m, y.m, v); });
+    each([](const Split3 &x, const Split3 &y, f32x4 v) { return PolBF16<64>::mma(x.m, y.h, v); });
+    each([](const Split3 &x, const Split3 &y, f32x4 v) { return PolBF16<64>::mma(x.h, y.m, v); });
+    each([](const Split3 &x, const Split3 &y, f32x4 v) { return PolBF16<64>::mma(x.h, y.h, v); });
+}
+
+// An fp32 64-row x 64 tile in LDS as its three parts, each in PolBF16<64>'s
+// layout (24 KB).
+struct SplitTile {
+    using Pol = PolBF16<64>;
+    __attribute__((aligned(16))) u16 part[3][Pol::ROWS * 64];
+
+    // operand rows n (score products): k-steps 0 and 1
+    __device__ __forceinline__ void row_frags(Split3 (&f)[2], int n, int g) const {
+        bf16x8 t[3][2];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) Pol::lds_row_frags(t[i], part[i], n, g);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) f[k] = Split3{t[0][k], t[1][k], t[2][k]};
+    }
+    // operand of the chained product: columns y0.. of the 32 rows from blk, transposed
+    __device__ __forceinline__ Split3 chain_a(int y0, int blk, int g, int l16) const {
+        return Split3{Pol::chain_a(part[0], y0, blk, g, l16), Pol::chain_a(part[1], y0, blk, g, l16),
+                      Pol::chain_a(part[2], y0, blk, g, l16)};
+    }
+};
+
+// One thread's share of a 64-row fp32 tile on its way to a SplitTile: chunk
+// positions k NT + tid of each part, 8 elements of one row each.
+template <int NT>
+struct SplitStage {
+    static constexpr int NK = 512 / NT;
+    f32x4 x[NK][2];
+    __device__ __forceinline__ void load(int k, const float *src) {
+        x[k][0] = *reinterpret_cast<const f32x4 *>(src);
+        x[k][1] = *reinterpret_cast<const f32x4 *>(src + 4);
+    }
+    __device__ __forceinline__ void write(SplitTile &t, int tid) const {
+#pragma unroll
+        for (int k = 0; k < NK; ++k) {
+            const Split3 s = split3(x[k][0], x[k][1]);
+            const int off = (k * NT + tid) * 8;
+            *reinterpret_cast<bf16x8 *>(t.part[0] + off) = s.h;
+            *reinterpret_cast<bf16x8 *>(t.part[1] + off) = s.m;
+            *reinterpret_cast<bf16x8 *>(t.part[2] + off) = s.l;
+        }
+    }
+};
+
 // --------------------------------------------------------------- LDS staging
 
 // Wave-wide direct global->LDS loads (global_load_lds_dwordx4 / _dword: no
