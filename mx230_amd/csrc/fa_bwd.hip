@@ -131,7 +131,7 @@ constexpr int kFlagRows = 128;  // query rows per flag: one dQ work-group's bloc
 // priority and the softmax part at normal priority (the one-launch backward,
 // where dQ and dK/dV waves share each SIMD).
 
-// 16x16 MFMA tiles (Pol = PolF32<64> or PolBF16<128>): lane l holds column
+// 16x16 MFMA tiles (bf16): lane l holds column
 // l%16 and rows 4(l/16) + r of each 16x16 C tile. W2 (bf16 d = 64, the
 // one-launch backward of small grids): compiled for two waves per SIMD, with
 // the stages' LDS operands read ahead of their products (stage_batched).
@@ -194,10 +194,9 @@ struct DqTile16 {
             }
 #pragma unroll
             for (int kc = 0; kc < NC; ++kc) {
-                if (!Pol::kExactScale) qf[qt][kc] = Pol::scaled(qf[qt][kc], p.scale_log2);
                 dof[qt][kc] = Pol::neg(dof[qt][kc]);
             }
-            nL2[qt] = ok ? lse[qt] * (Pol::kExactScale ? -1.0f / p.scale : -kLog2e) : 0.f;
+            nL2[qt] = ok ? lse[qt] * (-1.0f / p.scale) : 0.f;
         }
 #pragma unroll
         for (int xt = 0; xt < XT; ++xt) {
@@ -252,10 +251,8 @@ struct DqTile16 {
         sd[lane] = acc;
     }
 
-    // The score accumulators start at nL2, so they come out as the exponents
-    // of P, times xmul where the policy keeps Q exact (Pol::kExactScale: qf
-    // holds Q, nL2 is -L / scale, xmul = scale log2(e)); otherwise qf holds
-    // Q scale log2(e) and nL2 is -L log2(e).
+    // The score accumulators start at nL2 = -L / scale (qf holds Q itself), so
+    // times xmul = scale log2(e) they come out as the exponents of P.
     template <bool CAUSAL, bool MASK, bool PRIO>
     __device__ __forceinline__ void stage(const T *sk, const T *sv, int k0, int q0, int N, int lane, float xmul) {
         if constexpr (kBatchedReads) {
@@ -301,7 +298,7 @@ struct DqTile16 {
                             const int key = k0 + 32 * blk + Pol::bidx(t, g, r);
                             x = (key >= N || (CAUSAL && key > qi)) ? -INFINITY : x;
                         }
-                        const float pv = fast_exp2(Pol::kExactScale ? x * xmul : x);
+                        const float pv = fast_exp2(x * xmul);
                         s[t][qt][r] = pv * dp[t][qt][r];  // -dS / scale
                     }
                 }
@@ -374,7 +371,7 @@ struct DqTile16 {
                             const int key = k0 + 32 * blk + Pol::bidx(t, g, r);
                             x = (key >= N || (CAUSAL && key > qi)) ? -INFINITY : x;
                         }
-                        const float pv = fast_exp2(Pol::kExactScale ? x * xmul : x);
+                        const float pv = fast_exp2(x * xmul);
                         s[t][qt][r] = pv * dp[t][qt][r];  // -dS / scale
                     }
                 }
@@ -397,17 +394,10 @@ struct DqTile16 {
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt) {
             const int qi = q0 + 16 * qt + l16;
-            if constexpr (std::is_same<T, u16>::value) {
-                // bf16 rows, 16 bytes per lane
-                const size_t row = (size_t)min(qi, N - 1) * D;
+            const size_t row = (size_t)min(qi, N - 1) * D;  // 16 bytes per lane
 #pragma unroll
-                for (int xt = 0; xt < XT; xt += 2)
-                    store8_pair_bf16(dQ + row, 16 * xt, g, acc[xt][qt], acc[xt + 1][qt], -p.scale, qi < N);
-            } else if (qi < N) {
-#pragma unroll
-                for (int xt = 0; xt < XT; ++xt)
-                    store4<T>(dQ + (size_t)qi * D + 16 * xt + 4 * g, acc[xt][qt], -p.scale);
-            }
+            for (int xt = 0; xt < XT; xt += 2)
+                store8_pair_bf16(dQ + row, 16 * xt, g, acc[xt][qt], acc[xt + 1][qt], -p.scale, qi < N);
         }
     }
 };
@@ -453,13 +443,11 @@ struct DkvTile16 {
             for (int kc = 0; kc < NC; ++kc) {
                 if constexpr (P2) {
                     kf[kt][kc] = Pol::scaled(kf[kt][kc], -p.scale);
-                } else if constexpr (!Pol::kExactScale) {
-                    kf[kt][kc] = Pol::scaled(kf[kt][kc], p.scale_log2);
                 }
                 vf[kt][kc] = Pol::neg(vf[kt][kc]);
             }
         }
-        lmul = Pol::kExactScale ? -1.0f / p.scale : -kLog2e;
+        lmul = -1.0f / p.scale;
         xmul = P2 ? -kLog2e : p.scale_log2;
 #pragma unroll
         for (int xt = 0; xt < XT; ++xt) {
@@ -468,11 +456,9 @@ struct DkvTile16 {
         }
     }
 
-    // The score accumulators start at L lmul, so they come out as the
-    // exponents of P, times xmul where the policy keeps K exact
-    // (Pol::kExactScale: kf holds K, lmul = -1 / scale, xmul = scale
-    // log2(e)); otherwise kf holds K scale log2(e) and lmul = -log2(e). With
-    // P2 they start at L and kf holds -K scale, xmul = -log2(e).
+    // The score accumulators start at L lmul, lmul = -1 / scale (kf holds K
+    // itself), so times xmul = scale log2(e) they come out as the exponents of
+    // P. With P2 they start at L and kf holds -K scale, xmul = -log2(e).
     template <bool CAUSAL, bool MASK, bool PRIO>
     __device__ __forceinline__ void stage(const T *sq, const T *sdo, const float *sl, const float *sd, int qs, int kw0,
                                           int lane) {
@@ -517,7 +503,7 @@ struct DkvTile16 {
                 for (int r = 0; r < 4; ++r) {
 #pragma unroll
                     for (int kt = 0; kt < KT; ++kt) {
-                        float x = Pol::kExactScale || P2 ? s[t][kt][r] * xmul : s[t][kt][r];
+                        float x = s[t][kt][r] * xmul;
                         if constexpr (MASK) {
                             // causal: query qs + 32 blk + bidx(t, g, r) before key kw0 + 16 kt + l16
                             const bool before = Pol::bidx(t, g, r) - l16 < kw0 - qs + 16 * kt - 32 * blk;
@@ -607,7 +593,7 @@ struct DkvTile16 {
                 for (int r = 0; r < 4; ++r) {
 #pragma unroll
                     for (int kt = 0; kt < KT; ++kt) {
-                        float x = Pol::kExactScale || P2 ? s[t][kt][r] * xmul : s[t][kt][r];
+                        float x = s[t][kt][r] * xmul;
                         if constexpr (MASK) {
                             const bool before = Pol::bidx(t, g, r) - l16 < kw0 - qs + 16 * kt - 32 * blk;
                             x = before ? -INFINITY : x;
@@ -1129,6 +1115,377 @@ __device__ __forceinline__ void bwd_fused_entry(const Params &p) {
     }
 }
 
+// ------------------------------------------------- fp32 passes in bf16 parts
+
+// The fp32 passes (d = 64) with their products in bf16 parts (Split3): 4
+// waves, 64 rows per work-group (16 per wave, in registers as parts), 64 rows
+// of the other side per stage. Those pass through registers, loaded one stage
+// ahead, and are split once per work-group into one 48 KB LDS buffer. The dQ
+// pass holds three work-groups per CU (156 VGPRs), the dK/dV pass two (252),
+// whose splitting, softmax and matrix products overlap.
+//
+// Bound: the matrix unit and what of the splitting it does not hide. A wave's
+// stage is 144 (dQ) or 192 (dK/dV) MFMAs of 16 cycles, each hiding two VALU
+// instructions, and about 340 or 390 VALU instructions, 264 and 352 of them
+// splits. Event medians on one card, us, against v_mfma_f32_16x16x4_f32 (dQ /
+// dK/dV): causal B4 H12 N1024 107 / 146 -> 74 / 94, B4 H12 N4096 1161 / 1651
+// -> 755 / 1050, non-causal B1 H12 N4096 581 / 1026 -> 391 / 560, B1 H1 N256
+// 21.4 / 40.0 -> 17.9 / 20.5 (64 keys per work-group instead of 128). Errors of
+// dQ, dK, dV against 64 bits at the first: 1.0e-6, 1.2e-6, 1.1e-6 -> 3.7e-7,
+// 6.3e-7, 6.2e-7. The dQ pass at two work-groups per CU with both score tiles'
+// operands read at once: 76 / 798; the dK/dV pass at three spills 78 registers
+// (274 at B4 H12 N1024).
+struct SplitPair {
+    SplitTile a, b;
+};
+
+// The work-group's rows again in plain fp32 arithmetic, for operands outside
+// the parts' range: thread t takes elements 16 (t % 4) .. + 15 of row t / 4.
+template <bool CAUSAL>
+__device__ __forceinline__ void dq_plain(const Params &p, int bh, int qb) {
+    constexpr int D = 64;
+    const int qi = qb * 64 + (int)(threadIdx.x >> 2), c = 16 * (int)(threadIdx.x & 3);
+    const int b = bh / p.Hq, kvh = bh % p.Hq / p.group, row = min(qi, p.N - 1);
+    const size_t qoff = ((size_t)bh * p.N + row) * D + c, kvoff = ((size_t)b * p.Hkv + kvh) * p.N * D + c;
+    const float *K = static_cast<const float *>(p.k) + kvoff, *V = static_cast<const float *>(p.v) + kvoff;
+    float q[16], g[16], acc[16];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        q[e] = static_cast<const float *>(p.q)[qoff + e] * p.scale_log2;
+        g[e] = static_cast<const float *>(p.dout)[qoff + e];
+        acc[e] = 0.f;
+    }
+    const float l = p.lse[(size_t)bh * p.N + row] * kLog2e;
+    const float delta = p.o_in != nullptr ? dot16(g, static_cast<const float *>(p.o_in) + qoff)
+                                          : p.delta[(size_t)bh * p.N + row];
+    const int kend = CAUSAL ? row + 1 : p.N;
+    for (int k = 0; k < kend; ++k) {  // the 4 threads of a row share kend
+        const float ds = fast_exp2(dot16(q, K + (size_t)k * D) - l) * (dot16(g, V + (size_t)k * D) - delta);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[e] = __builtin_fmaf(ds, K[(size_t)k * D + e], acc[e]);
+    }
+    if (qi >= p.N) return;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) static_cast<float *>(p.dq)[qoff + e] = acc[e] * p.scale;
+}
+
+// dK (unscaled, sign flipped, times kmul) and dV of the work-group's 64 keys
+// over stages [g0, g0 + nsteps) of the group's query heads (dkv_split_entry).
+template <bool CAUSAL>
+__device__ __forceinline__ void dkv_plain(const Params &p, int bkv, int kb, int g0, int nsteps, float *dK, float *dV,
+                                       float kmul) {
+    constexpr int D = 64;
+    const int key = kb * 64 + (int)(threadIdx.x >> 2), c = 16 * (int)(threadIdx.x & 3), N = p.N;
+    const int row = min(key, N - 1), qstart = CAUSAL ? kb * 64 : 0, nqs = (N - qstart + 63) / 64;
+    const size_t koff = ((size_t)bkv * N + row) * D + c;
+    float k[16], v[16], ak[16], av[16];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        k[e] = static_cast<const float *>(p.k)[koff + e] * p.scale_log2;
+        v[e] = static_cast<const float *>(p.v)[koff + e];
+        ak[e] = av[e] = 0.f;
+    }
+    for (int st = g0; st < g0 + nsteps; ++st) {
+        const size_t bh = (size_t)(bkv / p.Hkv) * p.Hq + (size_t)(bkv % p.Hkv) * p.group + st / nqs;
+        const int q0 = qstart + st % nqs * 64;
+        for (int i = CAUSAL ? max(q0, row) : q0; i < min(q0 + 64, N); ++i) {
+            const size_t r = bh * N + i;
+            const float *Q = static_cast<const float *>(p.q) + r * D + c;
+            const float *G = static_cast<const float *>(p.dout) + r * D + c;
+            const float pv = fast_exp2(dot16(k, Q) - p.lse[r] * kLog2e), ds = pv * (p.delta[r] - dot16(v, G));
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                av[e] = __builtin_fmaf(pv, G[e], av[e]);
+                ak[e] = __builtin_fmaf(ds, Q[e], ak[e]);
+            }
+        }
+    }
+    if (key >= N) return;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        dK[(size_t)key * D + c + e] = ak[e] * kmul;
+        dV[(size_t)key * D + c + e] = av[e];
+    }
+}
+
+// The fp32 dQ pass, grid (B Hq, 64-query blocks).
+template <bool CAUSAL, bool DELTA>
+__device__ __forceinline__ void dq_split_entry(const Params &p) {
+    constexpr int D = 64, XT = 4, BQ = 64, BK = 64;
+    using PL = PolBF16<64>;  // the parts' layout
+    using Stage = SplitStage<256>;
+    __shared__ SplitPair sm;
+    __shared__ uint32_t flags[4];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = lane >> 4, l16 = lane & 15, N = p.N;
+    const int nqb = (N + BQ - 1) / BQ;
+    const int i = (int)(blockIdx.y * gridDim.x + blockIdx.x);
+    const int rank = CAUSAL ? cu_order_wg(i, p.cu_run, p.cu_runs) : i;  // heaviest first, balanced per CU
+    const int qb = CAUSAL ? nqb - 1 - rank / (int)gridDim.x : rank / (int)gridDim.x;
+    const int bh = rank % (int)gridDim.x;
+    const int b = bh / p.Hq, kvh = bh % p.Hq / p.group;
+    const size_t kvoff = ((size_t)b * p.Hkv + kvh) * N * D;
+    const float *K = static_cast<const float *>(p.k) + kvoff, *V = static_cast<const float *>(p.v) + kvoff;
+    const int q0 = qb * BQ + wave * 16, qi = q0 + l16;
+    wg_time(0);
+    const int nsteps = ((CAUSAL ? min(N, qb * BQ + BQ) : N) + BK - 1) / BK;
+    wg_info(0, qb, nsteps);
+
+    int srow[Stage::NK], scol[Stage::NK];
+#pragma unroll
+    for (int k = 0; k < Stage::NK; ++k) {
+        PL::chunk_at(k * 256 + tid, srow[k], scol[k]);
+        scol[k] *= 8;
+    }
+    Stage xk, xv;
+    auto load = [&](int st) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < Stage::NK; ++k) {
+            const size_t off = (size_t)min(st * BK + srow[k], N - 1) * D + scol[k];
+            xk.load(k, K + off);
+            xv.load(k, V + off);
+        }
+    };
+    load(0);
+
+    const size_t qrow = (size_t)bh * N + min(qi, N - 1);
+    Split3 qf[2], gf[2];
+    split_row(qf, static_cast<const float *>(p.q) + qrow * D, g, p.scale_log2, qi < N);
+    split_row(gf, static_cast<const float *>(p.dout) + qrow * D, g, -1.0f, qi < N);
+    // added to the scores and to -dP (-dO in registers) once the products are
+    // summed, smallest first: fewer roundings at the size of LSE
+    const float nl = qi < N ? -p.lse[qrow] * kLog2e : 0.f;
+    float dl = 0.f;
+    if constexpr (DELTA) {
+        const float *o = static_cast<const float *>(p.o_in) + qrow * D, *d = static_cast<const float *>(p.dout) + qrow * D;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int c = 32 * (e >> 3) + 8 * g + (e & 7);
+            dl = __builtin_fmaf(d[c], o[c], dl);
+        }
+        dl = xg_sum(dl);
+        if (qi < N && g == 0) p.delta[qrow] = dl;
+    } else {
+        dl = p.delta[qrow];
+    }
+    dl = qi < N ? dl : 0.f;
+    f32x4 acc[XT];
+#pragma unroll
+    for (int xt = 0; xt < XT; ++xt) acc[xt] = zero4();
+
+    auto compute = [&](bool edge, int k0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int blk = 0; blk < 2; ++blk) {
+            f32x4 s[2][1], dp[2][1];
+            const Split3 bq[1][2] = {{qf[0], qf[1]}}, bg[1][2] = {{gf[0], gf[1]}};
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                s[t][0] = dp[t][0] = zero4();
+                Split3 a[1][2];
+                f32x4 c[1][1] = {{zero4()}};
+                sm.a.row_frags(a[0], 32 * blk + PL::arow(t, l16), g);
+                mma_split_tiles<2, 1, 1>(c, a, bq);
+                s[t][0] = c[0][0];
+                c[0][0] = zero4();
+                sm.b.row_frags(a[0], 32 * blk + PL::arow(t, l16), g);
+                mma_split_tiles<2, 1, 1>(c, a, bg);
+                dp[t][0] = c[0][0];
+            }
+            if (edge) {
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int key = k0 + 32 * blk + PL::bidx(t, g, r);
+                        if (key >= N || (CAUSAL && key > qi)) s[t][0][r] = -INFINITY;
+                    }
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) s[t][0][r] = fast_exp2(s[t][0][r] + nl) * (dp[t][0][r] + dl);  // -dS / scale
+            }
+            const Split3 ds[1] = {split3(s[0][0], s[1][0])};
+#pragma unroll
+            for (int xt = 0; xt < XT; ++xt) {
+                const Split3 kt[1] = {sm.a.chain_a(16 * xt, 32 * blk, g, l16)};
+                acc[xt] = mma_split<1>(kt, ds, acc[xt]);
+            }
+        }
+    };
+    // only the last stage is masked: the diagonal, or the end of the keys
+    for (int st = 0; st < nsteps; ++st) {
+        if (st > 0) barrier_lds();  // every wave is done with the stage before
+        xk.write(sm.a, tid);
+        xv.write(sm.b, tid);
+        if (st + 1 < nsteps) load(st + 1);
+        barrier_lds();
+        if (st == 0) wg_time(1);
+        compute(st + 1 == nsteps, st * BK);
+    }
+    wg_time(2);
+    float z = 0.f;
+#pragma unroll
+    for (int xt = 0; xt < XT; ++xt) z += zero_of(acc[xt]);
+    if (any_nonfinite<4>(z, flags, wave, lane)) {
+        dq_plain<CAUSAL>(p, bh, qb);
+    } else if (qi < N) {
+        float *row = static_cast<float *>(p.dq) + qrow * D;
+#pragma unroll
+        for (int xt = 0; xt < XT; ++xt) store4<float>(row + 16 * xt + 4 * g, acc[xt], -p.scale);
+    }
+    wg_time_after_stores();
+}
+
+// The fp32 dK/dV pass, a 1-D grid of dkv_work's work-groups (64 keys each).
+template <bool CAUSAL>
+__device__ __forceinline__ void dkv_split_entry(const Params &p) {
+    constexpr int D = 64, XT = 4, BKV = 64, BQ = 64;
+    using PL = PolBF16<64>;
+    using Stage = SplitStage<256>;
+    __shared__ SplitPair sm;
+    __shared__ __attribute__((aligned(16))) float sL[BQ], sD[BQ];
+    __shared__ uint32_t flags[4];
+    const DkvWork wk = dkv_work(p, blockIdx.x, BKV, BQ, CAUSAL);
+    if (wk.kb * BKV >= p.N) return;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = lane >> 4, l16 = lane & 15, N = p.N;
+    const int b = wk.bkv / p.Hkv, kvh = wk.bkv % p.Hkv;
+    const size_t kvoff = (size_t)wk.bkv * N * D;
+    const int kw0 = wk.kb * BKV + wave * 16, key = kw0 + l16;
+    wg_time(0);
+    const int qstart = CAUSAL ? wk.kb * BKV : 0;
+    const int nqs = (N - qstart + BQ - 1) / BQ;  // stages per query head
+    int g0 = 0, nsteps = p.group * nqs;          // the share's stages
+    if (wk.ns > 1) {
+        g0 = (int)((long long)wk.sp * nsteps / wk.ns);
+        nsteps = (int)((long long)(wk.sp + 1) * nsteps / wk.ns) - g0;
+    }
+    wg_info(1, wk.kb, nsteps);
+
+    int srow[Stage::NK], scol[Stage::NK];
+#pragma unroll
+    for (int k = 0; k < Stage::NK; ++k) {
+        PL::chunk_at(k * 256 + tid, srow[k], scol[k]);
+        scol[k] *= 8;
+    }
+    // the next stage to load: its head's first row and its place in the head
+    size_t ld_row = ((size_t)b * p.Hq + (size_t)kvh * p.group + g0 / nqs) * N;
+    int ld_i = g0 % nqs;
+    Stage xq, xg;
+    float xl = 0.f;  // waves 0 and 1: LSE and Delta of row `lane`
+    auto load = [&]() __attribute__((always_inline)) {
+        const int qs = qstart + ld_i * BQ;
+#pragma unroll
+        for (int k = 0; k < Stage::NK; ++k) {
+            const size_t off = (ld_row + min(qs + srow[k], N - 1)) * D + scol[k];
+            xq.load(k, static_cast<const float *>(p.q) + off);
+            xg.load(k, static_cast<const float *>(p.dout) + off);
+        }
+        // rows past N: LSE = +inf makes their p (and so dS) exactly 0
+        if (wave == 0) xl = qs + lane < N ? p.lse[ld_row + qs + lane] : INFINITY;
+        if (wave == 1) xl = p.delta[ld_row + min(qs + lane, N - 1)];
+        if (++ld_i == nqs) {
+            ld_i = 0;
+            ld_row += N;
+        }
+    };
+    if (nsteps > 0) load();
+    Split3 kf[2], vf[2];
+    const size_t krow = kvoff + (size_t)min(key, N - 1) * D;
+    split_row(kf, static_cast<const float *>(p.k) + krow, g, p.scale_log2, key < N);
+    split_row(vf, static_cast<const float *>(p.v) + krow, g, -1.0f, key < N);
+    f32x4 accK[XT], accV[XT];
+#pragma unroll
+    for (int xt = 0; xt < XT; ++xt) accK[xt] = accV[xt] = zero4();
+
+    // diag: the stage's first queries may precede the keys. One body with the
+    // masking behind a branch: two bodies spill.
+    auto compute = [&](bool diag, int qs) __attribute__((always_inline)) {
+#pragma unroll
+        for (int blk = 0; blk < 2; ++blk) {
+            f32x4 s[2][1], dp[2][1];
+            Split3 a[2][2];
+            const Split3 bk[1][2] = {{kf[0], kf[1]}}, bv[1][2] = {{vf[0], vf[1]}};
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                s[t][0] = dp[t][0] = zero4();
+                sm.a.row_frags(a[t], 32 * blk + PL::arow(t, l16), g);
+            }
+            mma_split_tiles<2, 2, 1>(s, a, bk);
+#pragma unroll
+            for (int t = 0; t < 2; ++t) sm.b.row_frags(a[t], 32 * blk + PL::arow(t, l16), g);
+            mma_split_tiles<2, 2, 1>(dp, a, bv);
+            if (CAUSAL && diag) {
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        if (PL::bidx(t, g, r) - l16 < kw0 - qs - 32 * blk) s[t][0][r] = -INFINITY;
+                    }
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const int q4 = 32 * blk + PL::bidx(t, g, 0);
+                const f32x4 nl = *reinterpret_cast<const f32x4 *>(sL + q4);
+                const f32x4 dl = *reinterpret_cast<const f32x4 *>(sD + q4);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float pv = fast_exp2(s[t][0][r] + nl[r]);
+                    s[t][0][r] = pv;
+                    dp[t][0][r] = pv * (dp[t][0][r] + dl[r]);  // -dS / scale
+                }
+            }
+            const Split3 cp[1] = {split3(s[0][0], s[1][0])}, cds[1] = {split3(dp[0][0], dp[1][0])};
+#pragma unroll
+            for (int xt = 0; xt < XT; ++xt) {
+                const Split3 gt[1] = {sm.b.chain_a(16 * xt, 32 * blk, g, l16)};
+                accV[xt] = mma_split<1>(gt, cp, accV[xt]);
+                const Split3 qt[1] = {sm.a.chain_a(16 * xt, 32 * blk, g, l16)};
+                accK[xt] = mma_split<1>(qt, cds, accK[xt]);
+            }
+        }
+    };
+    int pos = g0 % nqs;  // the stage's place in its query head; the head's first is its diagonal
+    for (int st = 0; st < nsteps; ++st) {
+        if (st > 0) barrier_lds();
+        xq.write(sm.a, tid);
+        xg.write(sm.b, tid);
+        if (wave == 0) sL[lane] = -xl * kLog2e;
+        if (wave == 1) sD[lane] = xl;
+        if (st + 1 < nsteps) load();
+        barrier_lds();
+        if (st == 0) wg_time(1);
+        const int qs = qstart + pos * BQ;
+        compute(pos == 0, qs);
+        if (++pos == nqs) pos = 0;
+    }
+    wg_time(2);
+    // a share's partial sums go to its planes, unscaled (dkv_reduce_body)
+    const bool part = p.dkv_split > 1;
+    const size_t plane = (size_t)p.B * p.Hkv * N * D;
+    float *dK = part ? p.dkv_ws + (size_t)wk.sp * plane + kvoff : static_cast<float *>(p.dk) + kvoff;
+    float *dV = part ? dK + (size_t)p.dkv_split * plane : static_cast<float *>(p.dv) + kvoff;
+    const float kmul = part ? 1.0f : -p.scale;
+    float z = 0.f;
+#pragma unroll
+    for (int xt = 0; xt < XT; ++xt) z += zero_of(accK[xt]) + zero_of(accV[xt]);
+    if (any_nonfinite<4>(z, flags, wave, lane)) {
+        dkv_plain<CAUSAL>(p, wk.bkv, wk.kb, g0, nsteps, dK, dV, kmul);
+    } else if (key < N) {
+#pragma unroll
+        for (int xt = 0; xt < XT; ++xt) {
+            store4<float>(dK + (size_t)key * D + 16 * xt + 4 * g, accK[xt], kmul);
+            store4<float>(dV + (size_t)key * D + 16 * xt + 4 * g, accV[xt], 1.0f);
+        }
+    }
+    wg_time_after_stores();
+}
+
 // dK / dV of a split dK/dV pass: for each key row, the sum of its key block's
 // shares' fp32 partial planes in share order (so the result is
 // deterministic), times -scale for dK. n4 = float4 groups per plane
@@ -1166,8 +1523,15 @@ using DkvB64P2 = DkvTile16<PolBF16<64>, 2, true>;
 using DqB64W2 = DqTile16<PolBF16<64>, PolBF16<64>::kDqTiles, true>;
 using DkvB64W2 = DkvTile16<PolBF16<64>, 2, false, true>;
 using DkvB64P2W2 = DkvTile16<PolBF16<64>, 2, true, true>;
-using DqF32 = DqTile16<PolF32<64>, PolF32<64>::kDqTiles>;
-using DkvF32 = DkvTile16<PolF32<64>, 2>;
+// fp32 (dq_split_entry, dkv_split_entry): the launchers' view of their tiles
+struct DqF32 {
+    static constexpr int ROWS = 16, kWaves = 3;
+};
+struct DkvF32 {
+    using Pol = PolBF16<64>;  // 64-row stages
+    using T = float;
+    static constexpr int ROWS = 16, D = 64, kWaves = 2;
+};
 using DqB128 = DqTile16<PolBF16<128>, PolBF16<128>::kDqTiles>;
 using DkvB128 = DkvTile16<PolBF16<128>, 1>;
 
@@ -1183,6 +1547,10 @@ using DkvB128 = DkvTile16<PolBF16<128>, 1>;
     }
 #define MXFA_DKV(NAME, TILE, CAUSAL)                                                                     \
     extern "C" __global__ __launch_bounds__(256, TILE::kWaves) void NAME(Params p) { dkv_entry<TILE, CAUSAL>(p); }
+#define MXFA_DQ_F(NAME, CAUSAL, DELTA)                                                                   \
+    extern "C" __global__ __launch_bounds__(256, DqF32::kWaves) void NAME(Params p) { dq_split_entry<CAUSAL, DELTA>(p); }
+#define MXFA_DKV_F(NAME, CAUSAL)                                                                         \
+    extern "C" __global__ __launch_bounds__(256, DkvF32::kWaves) void NAME(Params p) { dkv_split_entry<CAUSAL>(p); }
 #define MXFA_FUSED(NAME, DQT, DKVT, CAUSAL)                                                              \
     extern "C" __global__ __launch_bounds__(256, DKVT::kWaves < DQT::kWaves ? DKVT::kWaves : DQT::kWaves) void \
     NAME(Params p) {                                                                                     \
@@ -1204,18 +1572,18 @@ MXFA_DQ(mxfa_dq_b128_c, DqB128, true, false)
 MXFA_DQ(mxfa_dq_b128_c_d, DqB128, true, true)
 MXFA_DQ(mxfa_dq_b128_n, DqB128, false, false)
 MXFA_DQ(mxfa_dq_b128_n_d, DqB128, false, true)
-MXFA_DQ(mxfa_dq_f64_c, DqF32, true, false)
-MXFA_DQ(mxfa_dq_f64_c_d, DqF32, true, true)
-MXFA_DQ(mxfa_dq_f64_n, DqF32, false, false)
-MXFA_DQ(mxfa_dq_f64_n_d, DqF32, false, true)
+MXFA_DQ_F(mxfa_dq_f64_c, true, false)
+MXFA_DQ_F(mxfa_dq_f64_c_d, true, true)
+MXFA_DQ_F(mxfa_dq_f64_n, false, false)
+MXFA_DQ_F(mxfa_dq_f64_n_d, false, true)
 MXFA_DKV(mxfa_dkv_b64_c, DkvB64, true)
 MXFA_DKV(mxfa_dkv_b64_n, DkvB64, false)
 MXFA_DKV(mxfa_dkv_b64_c_p2, DkvB64P2, true)
 MXFA_DKV(mxfa_dkv_b64_n_p2, DkvB64P2, false)
 MXFA_DKV(mxfa_dkv_b128_c, DkvB128, true)
 MXFA_DKV(mxfa_dkv_b128_n, DkvB128, false)
-MXFA_DKV(mxfa_dkv_f64_c, DkvF32, true)
-MXFA_DKV(mxfa_dkv_f64_n, DkvF32, false)
+MXFA_DKV_F(mxfa_dkv_f64_c, true)
+MXFA_DKV_F(mxfa_dkv_f64_n, false)
 MXFA_FUSED(mxfa_bwd_b64_c, DqB64, DkvB64, true)
 MXFA_FUSED(mxfa_bwd_b64_n, DqB64, DkvB64, false)
 MXFA_FUSED(mxfa_bwd_b64_c_p2, DqB64, DkvB64P2, true)
@@ -1231,6 +1599,8 @@ MXFA_REDUCE(mxfa_dkv_reduce_f32, float)
 #undef MXFA_PREPROCESS
 #undef MXFA_DQ
 #undef MXFA_DKV
+#undef MXFA_DQ_F
+#undef MXFA_DKV_F
 #undef MXFA_FUSED
 #undef MXFA_REDUCE
 #endif
@@ -1388,13 +1758,12 @@ static hipError_t launch_dkv_reduce(const Params &p, int causal, hipStream_t str
 //    another, so the heaviest share is the launch's critical path: at cfg5
 //    d = 64 (B1 Hq32 Hkv4 N2048), one query head per share left key block 0's
 //    32 stages per share as the last work-groups to end, with most slots idle.
-template <class Tile>
-static void dkv_plan_t(Params &p, bool causal) {
+static void dkv_plan(Params &p, bool causal, int BKV, int waves) {
     p.dkv_split = p.dkv_min_shares = 1;
     p.dkv_share_stages = 1 << 30;
     if (p.group <= 1) return;
-    constexpr int BKV = 4 * Tile::ROWS, BQ = Tile::Pol::ROWS;
-    constexpr long long kSlots = 256LL * Tile::kWaves;
+    constexpr int BQ = 64;
+    const long long kSlots = 256LL * waves;
     const long long nbkv = (long long)p.B * p.Hkv, nkb = (p.N + BKV - 1) / BKV;
     int s = p.group;
     for (int c = 1; c < p.group; ++c) {
@@ -1424,10 +1793,29 @@ static void dkv_plan_t(Params &p, bool causal) {
     p.dkv_split = most;
 }
 
-// The work-groups of a dK/dV pass (dkv_work's order) with p's split.
 template <class Tile>
-static long long dkv_work_groups(const Params &p, bool causal) {
-    constexpr int BKV = 4 * Tile::ROWS, BQ = Tile::Pol::ROWS;
+static void dkv_plan_t(Params &p, bool causal) {
+    static_assert(Tile::Pol::ROWS == 64, "dkv_plan's stages");
+    dkv_plan(p, causal, 4 * Tile::ROWS, Tile::kWaves);
+    if constexpr (std::is_same<typename Tile::T, float>::value) {
+        // never more planes than 128-key blocks with one work-group per CU take
+        // (the workspace callers have sized since before the 64-key blocks)
+        Params wide = p;
+        dkv_plan(wide, causal, 128, 1);
+        const int cap = wide.dkv_split;
+        if (p.dkv_split > cap) {
+            const long long most_stages = (long long)p.group * ((p.N + 63) / 64);
+            p.dkv_split = cap;
+            p.dkv_min_shares = std::min(p.dkv_min_shares, cap);
+            p.dkv_share_stages = (int)std::max<long long>(p.dkv_share_stages, (most_stages + cap - 1) / cap);
+        }
+    }
+}
+
+// The work-groups of a dK/dV pass over blocks of BKV keys (dkv_work's order)
+// with p's split.
+static long long dkv_work_groups(const Params &p, bool causal, int BKV) {
+    constexpr int BQ = 64;
     const long long nbkv = (long long)p.B * p.Hkv, nkb = (p.N + BKV - 1) / BKV;
     if (p.dkv_split <= 1) return nbkv * nkb;
     long long n = 0;
@@ -1456,12 +1844,14 @@ static size_t dkv_planes_bytes(const Params &p, int d) {
 
 // The workspace of a split dK/dV pass: its planes, then the one-launch
 // backward's share flags (8 bytes per share, dkv_work's order); 0 without a
-// split.
+// split. fp32: of the plan dkv_plan_t keeps within.
 template <class Tile>
 static size_t dkv_workspace_bytes_t(Params p, bool causal) {
-    dkv_plan_t<Tile>(p, causal);
+    constexpr bool kF32 = std::is_same<typename Tile::T, float>::value;
+    const int bkv = kF32 ? 128 : 4 * Tile::ROWS;
+    dkv_plan(p, causal, bkv, kF32 ? 1 : Tile::kWaves);
     if (p.dkv_split <= 1) return 0;
-    return dkv_planes_bytes(p, Tile::D) + 8 * (size_t)dkv_work_groups<Tile>(p, causal);
+    return dkv_planes_bytes(p, Tile::D) + 8 * (size_t)dkv_work_groups(p, causal, bkv);
 }
 
 size_t dkv_workspace_bytes(const Params &p, int dtype_bf16, int d, int causal) {
@@ -1506,7 +1896,7 @@ static hipError_t launch_fused_k(Params p, int causal, hipStream_t stream) {
     if (p.dkv_split == 1) p.dkv_ws = nullptr;
     const long long nfb = (p.N + kFlagRows - 1) / kFlagRows;
     const long long ndq = (long long)p.B * p.Hq * nfb;
-    const long long ndkv = dkv_work_groups<typename K::Dkv>(p, causal != 0);
+    const long long ndkv = dkv_work_groups(p, causal != 0, 4 * K::Dkv::ROWS);
     if (ndq + ndkv > 0x7fffffffLL) return hipErrorInvalidValue;
     unsigned e = ++g_epoch;
     if (e == 0) e = ++g_epoch;  // 0 is the flags' initial value
@@ -1558,7 +1948,7 @@ static hipError_t launch_dkv_k(Params p, int causal, hipStream_t stream) {
     dkv_plan_t<Tile>(p, causal != 0);
     if (p.dkv_ws == nullptr) p.dkv_split = 1;
     if (p.dkv_split == 1) p.dkv_ws = nullptr;
-    const long long n = dkv_work_groups<Tile>(p, causal != 0);
+    const long long n = dkv_work_groups(p, causal != 0, 4 * Tile::ROWS);
     if (n > 0x7fffffffLL) return hipErrorInvalidValue;
     void *args[] = {&p};
     const KernelId id = K::kHasP2 && scale_is_pow2(p.scale) ? K::dkv_p2[causal ? 1 : 0] : K::dkv[causal ? 1 : 0];

@@ -4,17 +4,17 @@
 //   * A "tile" is a 16x16 MFMA output. Lane l of a wave holds column l%16 and
 //     rows 4*(l/16) + r, r = 0..3 (the C layout of every 16x16 MFMA).
 //   * A "block" is 32 consecutive keys (or queries): the reduction depth of one
-//     chained bf16 MFMA (16x16x32) or of eight fp32 MFMAs (16x16x4).
+//     chained bf16 MFMA (16x16x32).
 //   * The first GEMM of a chain (scores, dP) produces two 16-row tiles t = 0,1
 //     per block. Its A-operand rows are permuted (Pol::arow) so that the lane
 //     holding C element (t, r) of column c holds block row Pol::bidx(t, g, r),
 //     g = l/16. For bf16 that puts rows 8g..8g+7 in one lane, which is exactly
 //     one k-slice of the next MFMA: the scores feed the next GEMM (P*V, dS*K,
 //     P^T*dO, dS^T*Q) straight from registers, no shuffle.
-//   * LDS tiles are row form, [n][D] (rows = keys or queries), with 16-byte
-//     chunks XOR-swizzled per row. The chained GEMMs contract over n: bf16 reads
-//     their operand transposed with ds_read_b64_tr_b16, fp32 reads it one
-//     element at a time.
+//   * LDS tiles hold rows of D elements (rows = keys or queries), 16-byte chunks
+//     in PolBF16's order; fp32 tiles as their three bf16 parts (SplitTile). The
+//     chained GEMMs contract over the rows: their operand is read transposed
+//     with ds_read_b64_tr_b16.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -260,7 +260,6 @@ struct PolBF16 {
     // operand to bf16 instead puts an error of about |S log2(e)| 2^-9 into
     // every exponent, correlated along a row or a key, which grows with the
     // logits and reaches the outputs through LSE.
-    static constexpr bool kExactScale = true;
     static constexpr int kWaves = 2;
     static constexpr int kWavesFwdCausal = D == 64 ? 3 : 2;
     static constexpr int kWavesDq = D == 64 ? 3 : 2;
@@ -388,109 +387,6 @@ struct PolBF16 {
     }
 };
 
-// fp32 parity path: v_mfma_f32_16x16x4_f32.
-template <int D_>
-struct PolF32 {
-    static constexpr int D = D_;
-    using T = float;
-    using Frag = float;
-    static constexpr int EPC = 4;
-    static constexpr int NC = D / 4;
-    static constexpr int ROWS = 64;
-    // fp32 operands: the scale folds into the operand with a 2^-24 rounding
-    static constexpr bool kExactScale = false;
-    // the forward runs 64-query work-groups at two waves per SIMD (fa_fwd.hip)
-    static constexpr int kWaves = 2;
-    static constexpr int kWavesFwdCausal = 2;
-    // dQ pass: one 16-query tile per wave at two waves per SIMD (202 VGPRs);
-    // two tiles at one wave ran slower (B1 H1 N256 backward 70.8 -> 57.5 us,
-    // B4 H12 N1024 causal 244 -> 235, B1 H12 N4096 non-causal 1812 -> 1604).
-    // dK/dV keeps 32 keys per wave at one wave: 16 keys spill at two
-    static constexpr int kWavesDq = 2;
-    static constexpr int kDqTiles = 1;
-    static constexpr int kDqWavesPerGroup = 4;
-    static constexpr int kWavesDkv = 1;
-    static constexpr int kDkvBuffers = 2;
-
-    __device__ static __forceinline__ int arow(int t, int m) { return (t << 4) + m; }
-    __device__ static __forceinline__ int bidx(int t, int g, int r) { return (t << 4) + (g << 2) + r; }
-    // Row-major tiles, 16-byte chunks XOR-swizzled by the low row bits.
-    __device__ static __forceinline__ int rswz(int n) { return n & 7; }
-    __device__ static __forceinline__ int chunk_off(int row, int chunk) {
-        return row * (D * 4) + ((chunk ^ rswz(row)) << 4);
-    }
-    __device__ static __forceinline__ void chunk_at(int P, int &row, int &chunk) {
-        row = P / (D / 4);
-        chunk = (P % (D / 4)) ^ rswz(row);
-    }
-
-    __device__ static __forceinline__ f32x4 mma(Frag a, Frag b, f32x4 c) {
-        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-    }
-    // k-slot g of MFMA s <-> element (D/4)*g + s of the row
-    __device__ static __forceinline__ void lds_row_frags(Frag (&f)[NC], const T *tile, int n, int g) {
-#pragma unroll
-        for (int i = 0; i < NC / 4; ++i) {
-            const int chunk = (NC / 4) * g + i;
-            const float4 v = *reinterpret_cast<const float4 *>(tile + n * D + ((chunk ^ rswz(n)) * EPC));
-            f[4 * i + 0] = v.x;
-            f[4 * i + 1] = v.y;
-            f[4 * i + 2] = v.z;
-            f[4 * i + 3] = v.w;
-        }
-    }
-    __device__ static __forceinline__ void gmem_row_frags_if(Frag (&f)[NC], const T *row, int g, bool valid) {
-#pragma unroll
-        for (int j = 0; j < NC / 4; ++j) {
-            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (valid) v = *reinterpret_cast<const float4 *>(row + NC * g + 4 * j);
-            f[4 * j + 0] = v.x;
-            f[4 * j + 1] = v.y;
-            f[4 * j + 2] = v.z;
-            f[4 * j + 3] = v.w;
-        }
-    }
-    // row i of n rows (row stride rs elements), zeros for i >= n (n >= 1),
-    // branch-free as in PolBF16
-    __device__ static __forceinline__ void gmem_row_frags(Frag (&f)[NC], const T *rows, int i, int n, size_t rs,
-                                                          int g) {
-        const bool valid = i < n;
-        const T *row = rows + (size_t)(valid ? i : n - 1) * rs;
-#pragma unroll
-        for (int j = 0; j < NC / 4; ++j) {
-            const float4 v = *reinterpret_cast<const float4 *>(row + NC * g + 4 * j);
-            f[4 * j + 0] = valid ? v.x : 0.f;
-            f[4 * j + 1] = valid ? v.y : 0.f;
-            f[4 * j + 2] = valid ? v.z : 0.f;
-            f[4 * j + 3] = valid ? v.w : 0.f;
-        }
-    }
-    __device__ static __forceinline__ Frag neg(Frag f) { return -f; }
-    __device__ static __forceinline__ Frag scaled(Frag f, float s) { return f * s; }
-    __device__ static __forceinline__ float dot(Frag a, Frag b) { return a * b; }
-    // The chain operand of one 32-row block: the two C tiles themselves.
-    struct ChainB {
-        f32x4 c0, c1;
-    };
-    __device__ static __forceinline__ ChainB pack(const f32x4 &c0, const f32x4 &c1) { return ChainB{c0, c1}; }
-    // Other[y][n] = tile[n][y0 + y] read element-wise: the k-slot g of MFMA
-    // (t, r) is block row 16t + 4g + r, matching the C layout of the chain tiles.
-    __device__ static __forceinline__ f32x4 chain(f32x4 acc, const ChainB &b, const T *tile, int y0, int blk,
-                                                  int g, int l16) {
-        const int y = y0 + l16;
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int n = blk + (t << 4) + (g << 2) + r;
-                const float a = tile[n * D + (((y >> 2) ^ rswz(n)) << 2) + (y & 3)];
-                acc = mma(a, t ? b.c1[r] : b.c0[r], acc);
-            }
-        }
-        return acc;
-    }
-};
-
 // ------------------------------------------------- fp32 products in bf16 parts
 
 // An fp32 value is the sum of three bf16 values h + m + l (each the nearest
@@ -506,10 +402,9 @@ struct Split3 {
 };
 
 //
-// The parts of an infinity, or of a value that rounds to one in bf16, are NaN
-// (inf - inf), as are those of its neighbour in a pair; kernels that use them
-// check their results and, on any that is not finite, run the work-group again
-// with v_mfma_f32_16x16x4_f32.
+// The later parts of an infinity, or of a value that rounds to one in bf16,
+// are NaN (inf - inf): kernels that use parts check their results and, on any
+// that is not finite, run the work-group again in plain fp32 arithmetic.
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 // One part of a pair: the nearest bf16s, packed, and what is left of each
@@ -964,6 +859,44 @@ __device__ __forceinline__ void wait_vmcnt() {
 template <class Pol, int NT = 256>
 constexpr int tile_loads() {
     return Pol::ROWS * (Pol::D / Pol::EPC) / NT;
+}
+
+// A row's two 8-element operands of a lane (k-steps 0 and 1), times mul, as
+// parts; zeros for rows that are not there.
+__device__ __forceinline__ void split_row(Split3 (&f)[2], const float *row, int g, float mul, bool valid) {
+#pragma unroll
+    for (int kc = 0; kc < 2; ++kc) {
+        const f32x4 a = *reinterpret_cast<const f32x4 *>(row + 32 * kc + 8 * g) * mul;
+        const f32x4 b = *reinterpret_cast<const f32x4 *>(row + 32 * kc + 8 * g + 4) * mul;
+        f[kc] = split3(valid ? a : zero4(), valid ? b : zero4());
+    }
+}
+
+// True for every wave of the work-group if any of its lanes holds a value that
+// is not finite (z: a sum of 0 x value, NaN then). A barrier inside.
+template <int NW>
+__device__ __forceinline__ bool any_nonfinite(float z, uint32_t *flags, int wave, int lane) {
+    const bool mine = __builtin_amdgcn_ballot_w64(z != 0.f) != 0;
+    if (lane == 0) flags[wave] = mine;
+    barrier_lds();
+    uint32_t any = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) any |= flags[w];
+    return __builtin_amdgcn_readfirstlane(any) != 0;
+}
+__device__ __forceinline__ float zero_of(f32x4 v) { return 0.f * v[0] + 0.f * v[1] + 0.f * v[2] + 0.f * v[3]; }
+
+// Plain fp32 arithmetic for those: a row's dot product, 16 elements in each of
+// the 4 consecutive lanes that share it.
+__device__ __forceinline__ float quad_sum(float x) {
+    x += __shfl_xor(x, 1, 4);
+    return x + __shfl_xor(x, 2, 4);
+}
+__device__ __forceinline__ float dot16(const float (&a)[16], const float *b) {
+    float s = 0.f;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) s = __builtin_fmaf(a[e], b[e], s);
+    return quad_sum(s);
 }
 
 // Store four consecutive elements x0..x0+3 of one output row.

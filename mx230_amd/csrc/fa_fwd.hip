@@ -13,8 +13,8 @@
 //     cross-lane reduction (two permlane swaps);
 //   * the output is accumulated transposed, O^T = V^T P^T, so the per-query
 //     rescale factor is a per-lane scalar as well;
-//   * exponentials are base 2: the fp32 scores are multiplied by
-//     scale log2(e) (bf16, which keeps Q exact) or Q is (fp32);
+//   * exponentials are base 2: the fp32 scores are multiplied by scale
+//     log2(e) (bf16, which keeps Q exact) or Q is (fp32, fwd_split_entry);
 //   * after the first stage the running max is only raised (and O and the sum
 //     rescaled) when some p of a row exceeds 2^16 (fwd_stage_lazy), detected
 //     from the per-lane row sums without computing a row maximum;
@@ -41,8 +41,8 @@ __device__ __forceinline__ constexpr int fwd_mask_offset(int blk, int t, int g, 
     return 32 * blk + Pol::bidx(t, g, r) - Pol::bidx(0, g, 0);
 }
 
-// One 64-key stage for one wave: scores in log2 units (x xmul when Q is kept
-// exact, else qf holds Q scale log2(e)), online-softmax update,
+// One 64-key stage for one wave: scores in log2 units (x xmul: qf holds Q
+// itself), online-softmax update,
 // O^T += V^T P^T. PRIO: the matrix products run at raised wave priority.
 // qpos0: position of the wave's first query row; Nk: key rows. EMPTY_ROWS:
 // rows may have every key of the stage masked (a key split's first stage).
@@ -81,7 +81,7 @@ __device__ __forceinline__ void fwd_stage(f32x4 (&acc)[Pol::D / 16][QT], float (
             for (int t = 0; t < 2; ++t) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    float v = Pol::kExactScale ? s[blk][t][qt][r] * xmul : s[blk][t][qt][r];
+                    float v = s[blk][t][qt][r] * xmul;
                     if constexpr (MASK) v = fwd_mask_offset<Pol>(blk, t, g, r) > lim ? -INFINITY : v;
                     s[blk][t][qt][r] = v;
                     mx = fmaxf(mx, v);
@@ -148,15 +148,15 @@ __device__ __forceinline__ void fwd_stage(f32x4 (&acc)[Pol::D / 16][QT], float (
 constexpr float kLazySum = 65536.0f;
 
 // Scores of one 64-key stage relative to m: s = K Q^T scale log2(e) - m, with
-// masked keys (MASK) at -inf. With Pol::kExactScale the accumulators start at
-// -m / xmul and the fp32 result is multiplied by xmul = scale log2(e).
+// masked keys (MASK) at -inf: the accumulators start at -m / xmul and the
+// fp32 result is multiplied by xmul = scale log2(e).
 template <class Pol, int QT, bool CAUSAL, bool MASK, bool PRIO = false>
 __device__ __forceinline__ void fwd_scores(f32x4 (&s)[2][2][QT], const float (&m)[QT],
                                            const typename Pol::Frag (&qf)[QT][Pol::NC], const typename Pol::T *sk,
                                            int k0, int qpos0, int Nk, int g, int l16, float xmul) {
     using Frag = typename Pol::Frag;
     constexpr int NC = Pol::NC;
-    const float im = Pol::kExactScale ? 1.0f / xmul : 1.0f;
+    const float im = 1.0f / xmul;
     f32x4 nm[QT];
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
@@ -175,7 +175,7 @@ __device__ __forceinline__ void fwd_scores(f32x4 (&s)[2][2][QT], const float (&m
                 f32x4 c = nm[qt];
 #pragma unroll
                 for (int kc = 0; kc < NC; ++kc) c = Pol::mma(a[kc], qf[qt][kc], c);
-                s[blk][t][qt] = Pol::kExactScale ? c * xmul : c;
+                s[blk][t][qt] = c * xmul;
             }
         }
     }
@@ -292,26 +292,20 @@ __device__ __forceinline__ void fwd_stage_lazy(f32x4 (&acc)[Pol::D / 16][QT], fl
 // nsteps / S) of its query block's keys and writes its unnormalised O and
 // its rows' running max and sum to Params::fwd_part; fwd_merge adds the
 // splits.
-template <class Pol>
-struct FwdSmem {
-    __attribute__((aligned(16))) typename Pol::T sK[2][Pol::ROWS * Pol::D];
-    __attribute__((aligned(16))) typename Pol::T sV[2][Pol::ROWS * Pol::D];
-};
-
-template <class Pol, bool CAUSAL, int QT, bool PAGED = false, bool SPLIT = false, int NW = 4>
-__device__ __forceinline__ void fwd_body(const Params &p, FwdSmem<Pol> &sm) {
+template <class Pol, bool CAUSAL, int QT, bool PAGED = false, bool SPLIT = false>
+__device__ __forceinline__ void fwd_entry(const Params &p) {
     using T = typename Pol::T;
     using Frag = typename Pol::Frag;
     constexpr int D = Pol::D, NC = Pol::NC, XT = D / 16;
-    constexpr int BQ = 16 * NW * QT, BK = Pol::ROWS, NT = 64 * NW;
-    // bf16: the matrix products at raised wave priority, the softmax at normal
+    constexpr int BQ = 64 * QT, BK = Pol::ROWS;
+    // the matrix products at raised wave priority, the softmax at normal
     // (A/B on one box: cfg4 78.1 -> 74.3 us, cfg5 d = 128 51.0 -> 47.2,
     // non-causal B2 H12 N4096 112.2 -> 109.7; the 64-query d = 64 launches
     // lost 1-3% with it)
-    constexpr bool kPrio = Pol::kExactScale && (QT == 2 || D == 128);
+    constexpr bool kPrio = QT == 2 || D == 128;
 
-    auto &sK = sm.sK;
-    auto &sV = sm.sV;
+    __shared__ __attribute__((aligned(16))) T sK[2][BK * D];
+    __shared__ __attribute__((aligned(16))) T sV[2][BK * D];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -336,15 +330,6 @@ __device__ __forceinline__ void fwd_body(const Params &p, FwdSmem<Pol> &sm) {
     Frag qf[QT][NC];
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) Pol::gmem_row_frags(qf[qt], Q, q0 + 16 * qt + l16, N, p.q_rs, g);
-    // fp32: Q scale log2(e), so the scores come out of the MFMAs in log2
-    // units; bf16 keeps Q exact and scales the fp32 scores instead
-#pragma unroll
-    for (int qt = 0; qt < QT; ++qt) {
-#pragma unroll
-        for (int kc = 0; kc < NC; ++kc) {
-            if (!Pol::kExactScale) qf[qt][kc] = Pol::scaled(qf[qt][kc], p.scale_log2);
-        }
-    }
     f32x4 acc[XT][QT];
     float m[QT], lsum[QT];
 #pragma unroll
@@ -363,16 +348,16 @@ __device__ __forceinline__ void fwd_body(const Params &p, FwdSmem<Pol> &sm) {
     const int s_hi = SPLIT ? (int)((long long)(blockIdx.z + 1) * nsteps / gridDim.z) : nsteps;
     wg_info(2, qb, s_hi - s_lo);
 
-    const RowPlan<Pol, NT> plan(tid);
+    const RowPlan<Pol> plan(tid);
     // PAGED: the table entries of stage 0 now, then each stage fetches those
     // of the stage after the one it stages
-    PagedRows<Pol, NT> paged;
+    PagedRows<Pol> paged;
     auto stage_next = [&](T *sk, T *sv, int k0) __attribute__((always_inline)) {
         if constexpr (PAGED) {
             paged.stage(sk, sv, K, V, k0, Nk, p.bs_shift, plan, wave, p.kv_rs);
             if (k0 + BK < Nk) paged.fetch(p.block_table, p.bs_shift, k0 + BK, Nk, plan);
         } else {
-            stage_kv<Pol, NT>(sk, sv, K, V, k0, Nk, plan, wave, p.kv_rs);
+            stage_kv<Pol>(sk, sv, K, V, k0, Nk, plan, wave, p.kv_rs);
         }
     };
     if (!SPLIT || s_lo < s_hi) {
@@ -462,72 +447,89 @@ __device__ __forceinline__ void fwd_body(const Params &p, FwdSmem<Pol> &sm) {
         const int qi = q0 + 16 * qt + l16;
         const float ltot = xg_sum(lsum[qt]);
         const float inv = 1.0f / ltot;
-        if constexpr (std::is_same<T, u16>::value) {
-            // bf16 rows, 16 bytes per lane (rows start on 16-byte boundaries)
-            T *row = O + (size_t)min(qi, N - 1) * p.o_rs;
+        // 16 bytes per lane (rows start on 16-byte boundaries)
+        T *row = O + (size_t)min(qi, N - 1) * p.o_rs;
 #pragma unroll
-            for (int xt = 0; xt < XT; xt += 2)
-                store8_pair_bf16(row, 16 * xt, g, acc[xt][qt], acc[xt + 1][qt], inv, qi < N);
-        } else if (qi < N) {
-#pragma unroll
-            for (int xt = 0; xt < XT; ++xt) store4<T>(O + (size_t)qi * p.o_rs + 16 * xt + 4 * g, acc[xt][qt], inv);
-        }
+        for (int xt = 0; xt < XT; xt += 2)
+            store8_pair_bf16(row, 16 * xt, g, acc[xt][qt], acc[xt + 1][qt], inv, qi < N);
         if (qi < N && p.lse != nullptr && g == 0) p.lse[(size_t)bh * N + qi] = (m[qt] + fast_log2(ltot)) * kLn2;
     }
     wg_time_after_stores();
 }
 
-template <class Pol, bool CAUSAL, int QT, bool PAGED = false, bool SPLIT = false>
-__device__ __forceinline__ void fwd_entry(const Params &p) {
-    __shared__ FwdSmem<Pol> sm;
-    fwd_body<Pol, CAUSAL, QT, PAGED, SPLIT>(p, sm);
-}
-
-// The fp32 forward (d = 64) with its products in bf16 parts (Split3): NW waves,
-// 16 NW queries per work-group, 64 keys per stage. Waves 2i and 2i + 1 hold the
-// same 32 queries (two 16-query tiles) and take the even and the odd 32-key
-// block of every stage, each with its own running max, sum and O; the pair
-// merges them through LDS at the end. So each K and V operand read from LDS
-// serves two tiles, half the LDS reads per product of one tile per wave. K and V
-// pass through registers, where each element is split once per work-group,
-// beside the score products of the stage before; the parts of a stage take 48
-// KB of LDS, double-buffered: one work-group per CU, NW / 4 waves per SIMD.
+// The fp32 forward (d = 64) with its products in bf16 parts (Split3): NW waves
+// of 16 queries, 64 keys per stage. K and V pass through registers, loaded one
+// stage ahead, and are split once per work-group into one 48 KB LDS buffer;
+// NW = 4: three work-groups per CU (162 VGPRs), NW = 8: two (114 VGPRs), whose
+// splitting, softmax and products overlap.
 //
-// Bound: a wave's stage is 96 MFMAs (1536 cycles) and about 230 VALU
-// instructions, of which an MFMA hides two; the rest of the ~5700 cycles that
-// the two waves of a SIMD take is the softmax between barriers, where both
-// run VALU code and the matrix unit idles. Measured against the
-// v_mfma_f32_16x16x4_f32 form (64 queries, two work-groups per CU), event
-// medians on one card, us: causal B4 H12 N1024 79.5 -> 54.6, B4 H12 N4096
-// 805.7 -> 576.4, non-causal B1 H12 N4096 410.8 -> 338.5 (152 TFLOP/s), B1 H1
-// N256 16.0 -> 14.6; 500 tokens after 3584 at 14/2 heads, split, 88.1 ->
-// 50.0 a call. Error of O against 64 bits: 3.5e-7 -> 2.5e-7 and 5.1e-7 ->
-// 3.5e-7 at the first two. Other forms tried at B4 H12 N4096: 64 queries and
-// 4 waves with one buffer, two work-groups per CU, 636 us (each K and V
-// element is then split by twice as many work-groups); the barrier at the end
-// of the stage instead of before the softmax 571 against 568.
-struct FwdSplitTiles {
+// Bound: a wave's stage is 96 MFMAs (1536 cycles, each hiding two VALU
+// instructions), 48 KB of LDS reads and about 340 (NW = 4) or 250 VALU
+// instructions, over half of them the splitting. Event medians on one card,
+// us, against v_mfma_f32_16x16x4_f32 on the same tiles: causal B4 H12 N1024
+// 79.5 -> 54, B4 H12 N4096 806 -> 523 (197 TFLOP/s), non-causal B1 H12 N4096
+// 411 -> 318, B1 H1 N256 16.0 -> 14.1. Error of O against 64 bits, same
+// shapes: 3.5e-7 -> 3.0e-7, 5.1e-7 -> 4.5e-7, 1.2e-6 -> 1.1e-6, 4.4e-7 ->
+// 4.1e-7. Two 16-query tiles per wave, the waves in pairs over half a stage's
+// keys each (half the LDS reads) ran 54.6, 570, 338 and 14.6: 250 VGPRs leave
+// two waves per SIMD.
+struct FwdSplitSmem {
     SplitTile k, v;
+    uint32_t flags[8];
 };
-union FwdSplitSmem {
-    FwdSplitTiles t[2];
-    struct {
-        float acc[8][64][17];  // a wave's 16 values per lane for its partner (odd row length: no bank conflicts)
-        float ml[8][2][16];
-        uint32_t bad[8];
-    } merge;
-    FwdSmem<PolF32<64>> f32;  // the fallback's
-};
+
+// The work-group's rows again in plain fp32 arithmetic, for operands outside
+// the parts' range: thread t takes elements 16 (t % 4) .. + 15 of row t / 4.
+template <int NW, bool CAUSAL, bool PAGED, bool SPLIT>
+__device__ __forceinline__ void fwd_plain(const Params &p, int bh, int qb, int key0, int key1) {
+    constexpr int D = 64;
+    const int qi = qb * 16 * NW + (int)(threadIdx.x >> 2), c = 16 * (int)(threadIdx.x & 3), row = min(qi, p.N - 1);
+    const int b = bh / p.Hq, h = bh % p.Hq, kvh = h / p.group;
+    const float *Q = static_cast<const float *>(p.q) + b * p.q_bs + h * p.q_hs + (size_t)row * p.q_rs + c;
+    const size_t kvoff = b * p.kv_bs + kvh * p.kv_hs + c;
+    float q[16], acc[16], m = -INFINITY, l = 0.f;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        q[e] = Q[e] * p.scale_log2;
+        acc[e] = 0.f;
+    }
+    const int kend = min(key1, CAUSAL ? min(p.Nk, p.pos0 + row + 1) : p.Nk);  // the same for a row's 4 threads
+    for (int k = key0; k < kend; ++k) {
+        size_t r = k;
+        if constexpr (PAGED) r = ((size_t)p.block_table[k >> p.bs_shift] << p.bs_shift) + (k & ((1 << p.bs_shift) - 1));
+        const float *K = static_cast<const float *>(p.k) + kvoff + r * (size_t)p.kv_rs;
+        const float *V = static_cast<const float *>(p.v) + kvoff + r * (size_t)p.kv_rs;
+        const float s = dot16(q, K), mn = fmaxf(m, s), mref = mn == -INFINITY ? 0.f : mn;
+        const float corr = fast_exp2(m - mref), pv = fast_exp2(s - mref);
+        m = mn;
+        l = l * corr + pv;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[e] = __builtin_fmaf(pv, V[e], acc[e] * corr);
+    }
+    if (qi >= p.N) return;
+    if constexpr (SPLIT) {
+        const size_t rows = (size_t)gridDim.z * p.B * p.Hq * p.N;
+        const size_t r0 = ((size_t)blockIdx.z * p.B * p.Hq + bh) * p.N + qi;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) p.fwd_part[r0 * D + c + e] = acc[e];
+        if (c == 0) *reinterpret_cast<float2 *>(p.fwd_part + rows * D + 2 * r0) = make_float2(m, l);
+    } else {
+        float *O = static_cast<float *>(p.o) + b * p.o_bs + h * p.o_hs + (size_t)qi * p.o_rs + c;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) O[e] = acc[e] / l;
+        if (p.lse != nullptr && c == 0) p.lse[(size_t)bh * p.N + qi] = (m + fast_log2(l)) * kLn2;
+    }
+}
 
 template <int NW, bool CAUSAL, bool PAGED, bool SPLIT>
 __device__ __forceinline__ void fwd_split_entry(const Params &p) {
-    constexpr int D = 64, XT = 4, QT = 2, BQ = 16 * NW, BK = 64, NT = 64 * NW;
+    constexpr int D = 64, XT = 4, BQ = 16 * NW, BK = 64, NT = 64 * NW;
     using PL = PolBF16<64>;  // the parts' layout
+    using Stage = SplitStage<NT>;
     __shared__ FwdSplitSmem sm;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wq = wave >> 1, wk = wave & 1;
     const int g = lane >> 4, l16 = lane & 15;
     const int N = p.N, Nk = p.Nk, pos0 = p.pos0;
     const int nqb = (N + BQ - 1) / BQ;
@@ -536,22 +538,18 @@ __device__ __forceinline__ void fwd_split_entry(const Params &p) {
     const int bh = rank % (int)gridDim.x;
     const int qb = CAUSAL ? nqb - 1 - rank / (int)gridDim.x : rank / (int)gridDim.x;
     const int b = bh / p.Hq, h = bh % p.Hq, kvh = h / p.group;
-    const float *Q = static_cast<const float *>(p.q) + b * p.q_bs + h * p.q_hs;
     const size_t kvoff = b * p.kv_bs + kvh * p.kv_hs;
     const float *K = static_cast<const float *>(p.k) + kvoff;
     const float *V = static_cast<const float *>(p.v) + kvoff;
-    const int q0 = qb * BQ + wq * 32;
-    const int qpos0 = pos0 + q0;
+    const int q0 = qb * BQ + wave * 16, qi = q0 + l16;
     wg_time(0);
 
-    const int kend = CAUSAL ? min(Nk, pos0 + qb * BQ + BQ) : Nk;
-    const int nsteps = (kend + BK - 1) / BK;
+    const int nsteps = ((CAUSAL ? min(Nk, pos0 + qb * BQ + BQ) : Nk) + BK - 1) / BK;
     const int s_lo = SPLIT ? (int)((long long)blockIdx.z * nsteps / gridDim.z) : 0;
     const int s_hi = SPLIT ? (int)((long long)(blockIdx.z + 1) * nsteps / gridDim.z) : nsteps;
     wg_info(2, qb, s_hi - s_lo);
 
     // this thread's chunks of a tile: row and first column
-    using Stage = SplitStage<NT>;
     int srow[Stage::NK], scol[Stage::NK], blk[Stage::NK];
 #pragma unroll
     for (int k = 0; k < Stage::NK; ++k) {
@@ -582,242 +580,141 @@ __device__ __forceinline__ void fwd_split_entry(const Params &p) {
         load(s_lo);
     }
 
-    Split3 qf[QT][2];
+    Split3 qf[1][2];
+    split_row(qf[0], static_cast<const float *>(p.q) + b * p.q_bs + h * p.q_hs + (size_t)min(qi, N - 1) * p.q_rs, g,
+              p.scale_log2, qi < N);
+    f32x4 acc[XT];
 #pragma unroll
-    for (int qt = 0; qt < QT; ++qt) {
-        const int qi = q0 + 16 * qt + l16;
-        const float *row = Q + (size_t)min(qi, N - 1) * p.q_rs;
-#pragma unroll
-        for (int kc = 0; kc < 2; ++kc) {
-            const f32x4 a = *reinterpret_cast<const f32x4 *>(row + 32 * kc + 8 * g) * p.scale_log2;
-            const f32x4 c = *reinterpret_cast<const f32x4 *>(row + 32 * kc + 8 * g + 4) * p.scale_log2;
-            qf[qt][kc] = split3(qi < N ? a : zero4(), qi < N ? c : zero4());
-        }
-    }
-    f32x4 acc[XT][QT];
-    float m[QT], lsum[QT];
-#pragma unroll
-    for (int qt = 0; qt < QT; ++qt) {
-#pragma unroll
-        for (int xt = 0; xt < XT; ++xt) acc[xt][qt] = zero4();
-        m[qt] = -INFINITY;
-        lsum[qt] = 0.f;
-    }
+    for (int xt = 0; xt < XT; ++xt) acc[xt] = zero4();
+    float m = -INFINITY, lsum = 0.f;
 
-    // The wave's 32-key block of the stage at k0: the online softmax of
-    // fwd_stage (FIRST) or, after the wave's first block, fwd_stage_lazy's (the
-    // scores are kept, so a redo starts from them). A row that precedes every
-    // key of the wave's first block has m = -inf, and then precedes all the
-    // wave's later ones.
-    f32x4 s[2][QT];
-    Split3 av[XT];
-    // after the wave's first block the scores are relative to m (rows with m = -inf: to 0)
-    auto scores = [&](bool first, const FwdSplitTiles &t) __attribute__((always_inline)) {
+    // One stage: the online softmax of fwd_stage (FIRST) or, after the
+    // work-group's first stage, fwd_stage_lazy's: scores relative to m, and
+    // m raised only where a lane's sum of p passes kLazySum. A row that precedes
+    // every key of the first stage (a key split) has m = -inf, and then
+    // precedes all later ones too.
+    auto compute = [&](auto first, bool edge, int k0) __attribute__((always_inline)) {
+        constexpr bool FIRST = decltype(first)::value;
+        const float start = FIRST || m == -INFINITY ? 0.f : -m;
+        f32x4 s[2][2];
 #pragma unroll
-        for (int qt = 0; qt < QT; ++qt) {
-            const float c = first || m[qt] == -INFINITY ? 0.f : -m[qt];
-            s[0][qt] = s[1][qt] = f32x4{c, c, c, c};
+        for (int u = 0; u < 2; ++u) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                Split3 a[1][2];
+                f32x4 c[1][1] = {{f32x4{start, start, start, start}}};
+                sm.k.row_frags(a[0], 32 * u + PL::arow(t, l16), g);
+                mma_split_tiles<2, 1, 1>(c, a, qf);
+                s[u][t] = c[0][0];
+            }
         }
-        Split3 a[2][2];
+        if (edge) {
+            const int lim = (CAUSAL ? min(pos0 + qi, Nk - 1) : Nk - 1) - k0 - PL::bidx(0, g, 0);
 #pragma unroll
-        for (int u = 0; u < 2; ++u) t.k.row_frags(a[u], 32 * wk + PL::arow(u, l16), g);
-        mma_split_tiles<2, 2, QT>(s, a, qf);
-    };
-    // the operands of P V, read before the barrier, in flight during it
-    auto operands = [&](const FwdSplitTiles &t) __attribute__((always_inline)) {
-#pragma unroll
-        for (int xt = 0; xt < XT; ++xt) av[xt] = t.v.chain_a(16 * xt, 32 * wk, g, l16);
-    };
-    auto softmax_pv = [&](auto first, auto mask, int k0) __attribute__((always_inline)) {
-        constexpr bool FIRST = decltype(first)::value, MASK = decltype(mask)::value;
-        Split3 pf[QT];
-#pragma unroll
-        for (int qt = 0; qt < QT; ++qt) {
-            if constexpr (MASK) {
-                const int lim = (CAUSAL ? min(qpos0 + 16 * qt + l16, Nk - 1) : Nk - 1) - k0 - PL::bidx(0, g, 0);
+            for (int u = 0; u < 2; ++u) {
 #pragma unroll
                 for (int t = 0; t < 2; ++t) {
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) s[t][qt][r] = PL::bidx(t, 0, r) > lim ? -INFINITY : s[t][qt][r];
+                    for (int r = 0; r < 4; ++r) {
+                        if (32 * u + PL::bidx(t, 0, r) > lim) s[u][t][r] = -INFINITY;
+                    }
                 }
             }
         }
-        f32x4 pv[2][QT];
-        auto exps = [&](int qt, float sub) __attribute__((always_inline)) {
+        f32x4 pv[2][2];
+        auto exps = [&](float sub) __attribute__((always_inline)) {
             float ls = 0.f;
 #pragma unroll
-            for (int t = 0; t < 2; ++t) {
+            for (int u = 0; u < 2; ++u) {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float e = fast_exp2(s[t][qt][r] - sub);
-                    pv[t][qt][r] = e;
-                    ls += e;
+                for (int t = 0; t < 2; ++t) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float e = fast_exp2(s[u][t][r] - sub);
+                        pv[u][t][r] = e;
+                        ls += e;
+                    }
                 }
             }
             return ls;
         };
-        auto raise = [&](int qt) __attribute__((always_inline)) {  // m to the block's max, O and the sum rescaled
+        auto raise = [&]() __attribute__((always_inline)) {  // m to the stage's max, O and the sum rescaled
             float mx = -INFINITY;
 #pragma unroll
-            for (int t = 0; t < 2; ++t) {
+            for (int u = 0; u < 2; ++u) {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[t][qt][r]);
+                for (int t = 0; t < 2; ++t) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[u][t][r]);
+                }
             }
-            mx = xg_max(mx);  // relative to m after the first block
+            mx = xg_max(mx);  // relative to m after the first stage
             const float shift = FIRST ? (mx == -INFINITY ? 0.f : mx) : fmaxf(mx, 0.f);
-            const float corr = FIRST ? 0.f : fast_exp2(-shift);
-            m[qt] = FIRST ? mx : m[qt] + shift;
-            lsum[qt] *= corr;
+            m = FIRST ? mx : m + shift;
             if constexpr (!FIRST) {
+                const float corr = fast_exp2(-shift);
+                lsum *= corr;
 #pragma unroll
-                for (int xt = 0; xt < XT; ++xt) acc[xt][qt] *= corr;
+                for (int xt = 0; xt < XT; ++xt) acc[xt] *= corr;
             }
-            lsum[qt] += exps(qt, shift);
+            lsum += exps(shift);
         };
         if constexpr (FIRST) {
-#pragma unroll
-            for (int qt = 0; qt < QT; ++qt) raise(qt);
+            raise();
         } else {
-            float ls[QT];
-            bool over = false;
-#pragma unroll
-            for (int qt = 0; qt < QT; ++qt) {
-                ls[qt] = exps(qt, 0.f);
-                over = over || ls[qt] > kLazySum;
-            }
-            if (__builtin_amdgcn_ballot_w64(over) != 0) {
-#pragma unroll
-                for (int qt = 0; qt < QT; ++qt) raise(qt);
+            const float ls = exps(0.f);
+            if (__builtin_amdgcn_ballot_w64(ls > kLazySum) != 0) {
+                raise();
             } else {
-#pragma unroll
-                for (int qt = 0; qt < QT; ++qt) lsum[qt] += ls[qt];
+                lsum += ls;
             }
         }
 #pragma unroll
-        for (int qt = 0; qt < QT; ++qt) pf[qt] = split3(pv[0][qt], pv[1][qt]);
+        for (int u = 0; u < 2; ++u) {
+            const Split3 pf[1] = {split3(pv[u][0], pv[u][1])};
 #pragma unroll
-        for (int xt = 0; xt < XT; ++xt) {
-            const Split3 a[1] = {av[xt]};
-#pragma unroll
-            for (int qt = 0; qt < QT; ++qt) {
-                const Split3 bq[1] = {pf[qt]};
-                acc[xt][qt] = mma_split<1>(a, bq, acc[xt][qt]);
+            for (int xt = 0; xt < XT; ++xt) {
+                const Split3 a[1] = {sm.v.chain_a(16 * xt, 32 * u, g, l16)};
+                acc[xt] = mma_split<1>(a, pf, acc[xt]);
             }
         }
     };
-
-    // Stages that no wave masks first, then the rest (fwd_body's split of
-    // them). The wave's first stage is the work-group's first: a wave skips a
-    // stage only when all its keys follow the wave's queries, and then every
-    // later one.
-    const int nmain = min(min(s_hi, Nk / BK), CAUSAL ? (pos0 + qb * BQ + 1) / BK : s_hi);
-    // A stage: its scores, with the next stage's parts written beside them,
-    // and the reads of V; a barrier; softmax and P V, which run on into the next
-    // stage's scores. The barrier orders both the writes of stage st + 1 before
-    // its reads and the reads of stage st before stage st + 2's writes.
-    auto stage = [&](auto first, auto mask, int st) __attribute__((always_inline)) {
-        const int cur = (st - s_lo) & 1, k0 = st * BK + 32 * wk;
-        const bool live = !decltype(mask)::value || !CAUSAL || k0 <= qpos0 + 31;
-        if (live) scores(decltype(first)::value, sm.t[cur]);
-        if (st + 1 < s_hi) {
-            xk.write(sm.t[cur ^ 1].k, tid);
-            xv.write(sm.t[cur ^ 1].v, tid);
-            if (st + 2 < s_hi) load(st + 2);
-        }
-        if (live) operands(sm.t[cur]);
+    // stages from `nmain` on have keys that some wave masks; a wave whose
+    // queries all precede a stage's keys skips it, and every later one
+    const int nmain = min(Nk / BK, CAUSAL ? (pos0 + qb * BQ + 1) / BK : nsteps);
+    auto stage = [&](auto first, int st) __attribute__((always_inline)) {
+        if (st > s_lo) barrier_lds();  // every wave is done with the stage before
+        xk.write(sm.k, tid);
+        xv.write(sm.v, tid);
+        if (st + 1 < s_hi) load(st + 1);
         barrier_lds();
-        if (live) softmax_pv(first, mask, k0);
+        if (!CAUSAL || st * BK <= pos0 + q0 + 15) compute(first, st >= nmain, st * BK);
     };
-    if (s_lo < s_hi) {
-        xk.write(sm.t[0].k, tid);
-        xv.write(sm.t[0].v, tid);
-        if (s_lo + 1 < s_hi) load(s_lo + 1);
-    }
-    barrier_lds();
+    if (s_lo < s_hi) stage(std::true_type{}, s_lo);
     wg_time(1);
-    int st = s_lo;
-    if (st < nmain) stage(std::true_type{}, std::false_type{}, st++);
-    for (; st < nmain; ++st) stage(std::false_type{}, std::false_type{}, st);
-    if (st == s_lo && st < s_hi) stage(std::true_type{}, std::true_type{}, st++);
-    for (; st < s_hi; ++st) stage(std::false_type{}, std::true_type{}, st);
+    for (int st = s_lo + 1; st < s_hi; ++st) stage(std::false_type{}, st);
     wg_time(2);
-    barrier_lds();  // every wave is done with the tiles
 
-    // Each wave finishes one of the pair's two query tiles (wk): it gives the
-    // other tile's state to its partner and merges the partner's into its own.
-    float lt[QT];
+    const float ltot = xg_sum(lsum);
+    float z = 0.f * ltot;
 #pragma unroll
-    for (int qt = 0; qt < QT; ++qt) lt[qt] = xg_sum(lsum[qt]);
-    auto give = [&](auto tile) __attribute__((always_inline)) {
-        constexpr int G = decltype(tile)::value;
-#pragma unroll
-        for (int xt = 0; xt < XT; ++xt) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) sm.merge.acc[wave][lane][4 * xt + r] = acc[xt][G][r];
-        }
-        if (g == 0) {
-            sm.merge.ml[wave][0][l16] = m[G];
-            sm.merge.ml[wave][1][l16] = lt[G];
-        }
-    };
-    auto finish = [&](auto tile) __attribute__((always_inline)) {
-        constexpr int G = decltype(tile)::value;
-        const int qi = q0 + 16 * G + l16;
-        const float mo = sm.merge.ml[wave ^ 1][0][l16], lo = sm.merge.ml[wave ^ 1][1][l16];
-        const float M = fmaxf(m[G], mo), mref = M == -INFINITY ? 0.f : M;
-        const float wa = fast_exp2(m[G] - mref), wb = fast_exp2(mo - mref);
-        const float L = wa * lt[G] + wb * lo;
-        f32x4 o[XT];
-#pragma unroll
-        for (int xt = 0; xt < XT; ++xt) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                o[xt][r] = wa * acc[xt][G][r] + wb * sm.merge.acc[wave ^ 1][lane][4 * xt + r];
-        }
-        // anything not finite: the whole work-group again on the fp32 matrix
-        // instructions (the parts of an infinity are NaN)
-        float z = 0.f * L;
-#pragma unroll
-        for (int xt = 0; xt < XT; ++xt) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) z += 0.f * o[xt][r];
-        }
-        const bool nonfinite = __builtin_amdgcn_ballot_w64(z != 0.f) != 0;
-        if (lane == 0) sm.merge.bad[wave] = nonfinite;
-        barrier_lds();
-        uint32_t bad = 0;
-#pragma unroll
-        for (int w = 0; w < NW; ++w) bad |= sm.merge.bad[w];
-        if (__builtin_amdgcn_readfirstlane(bad) != 0) return true;
-        if (qi >= N) return false;
+    for (int xt = 0; xt < XT; ++xt) z += zero_of(acc[xt]);
+    if (any_nonfinite<NW>(z, sm.flags, wave, lane)) {
+        fwd_plain<NW, CAUSAL, PAGED, SPLIT>(p, bh, qb, s_lo * BK, s_hi * BK);
+    } else if (qi < N) {
         if constexpr (SPLIT) {
             const size_t rows = (size_t)gridDim.z * p.B * p.Hq * N;
             const size_t r0 = ((size_t)blockIdx.z * p.B * p.Hq + bh) * N + qi;
 #pragma unroll
-            for (int xt = 0; xt < XT; ++xt) store4<float>(p.fwd_part + r0 * D + 16 * xt + 4 * g, o[xt], 1.0f);
-            if (g == 0) *reinterpret_cast<float2 *>(p.fwd_part + rows * D + 2 * r0) = make_float2(M, L);
+            for (int xt = 0; xt < XT; ++xt) store4<float>(p.fwd_part + r0 * D + 16 * xt + 4 * g, acc[xt], 1.0f);
+            if (g == 0) *reinterpret_cast<float2 *>(p.fwd_part + rows * D + 2 * r0) = make_float2(m, ltot);
         } else {
             float *O = static_cast<float *>(p.o) + b * p.o_bs + h * p.o_hs + (size_t)qi * p.o_rs;
-            const float inv = 1.0f / L;
+            const float inv = 1.0f / ltot;
 #pragma unroll
-            for (int xt = 0; xt < XT; ++xt) store4<float>(O + 16 * xt + 4 * g, o[xt], inv);
-            if (p.lse != nullptr && g == 0) p.lse[(size_t)bh * N + qi] = (M + fast_log2(L)) * kLn2;
+            for (int xt = 0; xt < XT; ++xt) store4<float>(O + 16 * xt + 4 * g, acc[xt], inv);
+            if (p.lse != nullptr && g == 0) p.lse[(size_t)bh * N + qi] = (m + fast_log2(ltot)) * kLn2;
         }
-        return false;
-    };
-    using T0 = std::integral_constant<int, 0>;
-    using T1 = std::integral_constant<int, 1>;
-    if (wk == 0) {
-        give(T1{});
-    } else {
-        give(T0{});
-    }
-    barrier_lds();
-    const bool redo = wk == 0 ? finish(T0{}) : finish(T1{});
-    if (redo) {
-        barrier_lds();  // every wave has read the flags
-        fwd_body<PolF32<64>, CAUSAL, 1, PAGED, SPLIT, NW>(p, sm.f32);
-        return;
     }
     wg_time_after_stores();
 }
@@ -891,14 +788,17 @@ MXFA_FWD(mxfa_fwd_b128_c_w2_q1, PolBF16<128>, true, 2, 1)
 MXFA_FWD(mxfa_fwd_b128_n_w2_q2, PolBF16<128>, false, 2, 2)
 // fp32
 #define MXFA_FWD_F(NAME, NW, CAUSAL, PG, SP)                                                            \
-    extern "C" __global__ __launch_bounds__(64 * NW, NW / 4) void NAME(Params p) { fwd_split_entry<NW, CAUSAL, PG, SP>(p); }
-MXFA_FWD_F(mxfa_fwd_f64_c, 8, true, false, false)
-MXFA_FWD_F(mxfa_fwd_f64_n, 8, false, false, false)
-MXFA_FWD_F(mxfa_fwd_f64_c_g4, 4, true, false, false)
-MXFA_FWD_F(mxfa_fwd_f64_n_g4, 4, false, false, false)
-MXFA_FWD_F(mxfa_fwd_f64_c_pg, 8, true, true, false)
-MXFA_FWD_F(mxfa_fwd_f64_c_sp, 8, true, false, true)
-MXFA_FWD_F(mxfa_fwd_f64_c_pg_sp, 8, true, true, true)
+    extern "C" __global__ __launch_bounds__(64 * NW, NW == 8 ? 4 : 3) void NAME(Params p) {              \
+        fwd_split_entry<NW, CAUSAL, PG, SP>(p);                                                          \
+    }
+MXFA_FWD_F(mxfa_fwd_f64_c, 4, true, false, false)
+MXFA_FWD_F(mxfa_fwd_f64_n, 4, false, false, false)
+MXFA_FWD_F(mxfa_fwd_f64_c_g8, 8, true, false, false)
+MXFA_FWD_F(mxfa_fwd_f64_n_g8, 8, false, false, false)
+MXFA_FWD_F(mxfa_fwd_f64_c_pg, 4, true, true, false)
+MXFA_FWD_F(mxfa_fwd_f64_c_pg_g8, 8, true, true, false)
+MXFA_FWD_F(mxfa_fwd_f64_c_sp, 4, true, false, true)
+MXFA_FWD_F(mxfa_fwd_f64_c_pg_sp, 4, true, true, true)
 // the prefill over a paged cache (causal, as the prefill always is)
 // (the table entries take registers: the three-wave 128-query d = 64 and the
 // 128-query d = 128 forms would spill in their loops, so paged launches use
@@ -937,7 +837,7 @@ MXFA_FWD_MERGE(mxfa_fwd_merge32_f64, float, 64, kFwdMaxSplits)
 // bf16 only; fp32 goes through launch_fwd_f32.
 template <class Pol, bool CAUSAL>
 static KernelId fwd_kernel_id(int wps, int qt, bool paged) {
-    if constexpr (Pol::kExactScale && Pol::D == 64) {
+    if constexpr (Pol::D == 64) {
         if (CAUSAL && paged) return qt == 1 ? k_mxfa_fwd_b64_c_w3_q1_pg : k_mxfa_fwd_b64_c_w2_q2_pg;
         if (CAUSAL) return qt == 1 ? k_mxfa_fwd_b64_c_w3_q1 : wps == 3 ? k_mxfa_fwd_b64_c_w3_q2 : k_mxfa_fwd_b64_c_w2_q2;
         return qt == 1 ? k_mxfa_fwd_b64_n_w3_q1 : k_mxfa_fwd_b64_n_w2_q2;
@@ -979,7 +879,7 @@ static hipError_t launch_fwd_qt(Params p, hipStream_t stream) {
 // for the paged prefill to give the contiguous one's bits.
 template <class Pol, bool CAUSAL>
 static hipError_t launch_fwd_t(const Params &p, hipStream_t stream) {
-    if constexpr (Pol::kExactScale && (CAUSAL || Pol::D == 64)) {
+    if constexpr (CAUSAL || Pol::D == 64) {
         constexpr long long kSlots = 256LL * Pol::kWavesFwdCausal;
         const long long wg = (long long)p.B * p.Hq * ((p.N + 127) / 128);
         if (wg < kSlots || (Pol::D == 128 && p.prefill != 0))
@@ -988,39 +888,37 @@ static hipError_t launch_fwd_t(const Params &p, hipStream_t stream) {
     return launch_fwd_qt<Pol, CAUSAL, 2>(p, stream);
 }
 
-// The fp32 forward: 128-query work-groups of 8 waves, one to a CU; where they
-// would leave half the CUs idle, 64-query ones of 4 waves (the same waves and
-// the same bits, each work-group splitting its K and V for itself): B1 H1 N256
-// 18.0 -> 14.6 us.
-static hipError_t launch_fwd_f32(const Params &p, int causal, hipStream_t stream) {
-    const long long bh = (long long)p.B * p.Hq;
-    const int nw = p.block_table == nullptr && bh * ((p.N + 127) / 128) <= 128 ? 4 : 8;
+// The fp32 forward: 8 waves and 128 queries per work-group where those fill the
+// two that a CU holds (each K and V element is then split half as often: B4 H12
+// N4096 causal 590 -> 523 us); 4 waves and 64 queries on smaller grids (B4 H12
+// N1024 causal 60 -> 54, B1 H1 N256 16.8 -> 14.1; 384 of 128 queries, B1 H12
+// N4096, 310 and 318 non-causal, 192 both causal). The same waves, so the
+// same bits.
+static hipError_t launch_fwd_f32(Params p, int causal, hipStream_t stream) {
+    const bool pg = p.block_table != nullptr;
+    const int nw = (long long)p.B * p.Hq * ((p.N + 127) / 128) >= 512 ? 8 : 4;
     const dim3 grid(p.B * p.Hq, (p.N + 16 * nw - 1) / (16 * nw));
-    const KernelId id = p.block_table != nullptr ? k_mxfa_fwd_f64_c_pg
-                        : nw == 4                ? (causal ? k_mxfa_fwd_f64_c_g4 : k_mxfa_fwd_f64_n_g4)
-                                                 : (causal ? k_mxfa_fwd_f64_c : k_mxfa_fwd_f64_n);
-    Params q = p;
-    void *args[] = {&q};
+    const KernelId id = nw == 8 ? (pg ? k_mxfa_fwd_f64_c_pg_g8 : causal ? k_mxfa_fwd_f64_c_g8 : k_mxfa_fwd_f64_n_g8)
+                                : (pg ? k_mxfa_fwd_f64_c_pg : causal ? k_mxfa_fwd_f64_c : k_mxfa_fwd_f64_n);
+    if (causal && nw == 4) cu_balance(&p, id, (long long)grid.x * grid.y);
+    void *args[] = {&p};
     return launch_kernel(id, grid, dim3(64 * nw), args, stream);
 }
 
-// Splits of the prefill's keys: none (1) when the 64-query (fp32: 128-query)
-// work-groups already fill the resident slots (bf16: 256 CUs x waves per SIMD;
-// fp32: 256, one work-group to a CU, so the splits make one round of them and
-// no part of a second) halfway, or when
+// Splits of the prefill's keys: none (1) when the 64-query work-groups
+// already fill the resident slots (256 CUs x waves per SIMD) halfway, or when
 // the heaviest query block has under 16 key stages (bf16; 8 for fp32), where
 // the merging launch costs more than the split saves (measured on the MI355X,
 // Qwen2.5 heads, 512 tokens at position 0, 8 stages: bf16 19.7 -> 24.6 us
 // with 2 splits, fp32 36.5 -> 32.6 us); else enough to fill them, with at
 // least 2 key stages per split and at most kFwdMaxSplits splits.
 int fwd_splits(const Params &p, int dtype_bf16, int d) {
-    const int rows = dtype_bf16 ? 64 : 128;  // per work-group
-    const long long wgs = (long long)p.B * p.Hq * ((p.N + rows - 1) / rows);
-    const long long slots = 256LL * (!dtype_bf16 ? 1 : d == 64 ? 3 : 2);
+    const long long wgs = (long long)p.B * p.Hq * ((p.N + 63) / 64);
+    const long long slots = 256LL * (dtype_bf16 && d == 64 ? 3 : 2);
     if (2 * wgs >= slots) return 1;
     const long long stages = (std::min(p.Nk, p.pos0 + p.N) + 63) / 64;  // the heaviest block's
     if (stages < (dtype_bf16 ? 16 : 8)) return 1;
-    long long s = dtype_bf16 ? (slots + wgs - 1) / wgs : slots / wgs;  // fp32: one round of one work-group per CU
+    long long s = (slots + wgs - 1) / wgs;
     s = std::min(s, std::max(1LL, stages / 2));
     return (int)std::min(s, (long long)kFwdMaxSplits);
 }
@@ -1043,9 +941,7 @@ hipError_t launch_fwd_split(const Params &p, int dtype_bf16, int d, int splits, 
                                    : (m8 ? k_mxfa_fwd_merge8_f64 : k_mxfa_fwd_merge32_f64);
     Params q = p;
     void *args[] = {&q};
-    const int rows = dtype_bf16 ? 64 : 128;
-    hipError_t e = launch_kernel(kf, dim3(p.B * p.Hq, (p.N + rows - 1) / rows, splits), dim3(dtype_bf16 ? 256 : 512), args,
-                                 stream);
+    hipError_t e = launch_kernel(kf, dim3(p.B * p.Hq, (p.N + 63) / 64, splits), dim3(256), args, stream);
     if (e != hipSuccess) return e;
     const size_t n = (size_t)p.B * p.Hq * p.N * (d / 4);
     int s = splits;

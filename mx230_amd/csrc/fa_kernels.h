@@ -7,7 +7,7 @@
 // the code object fails that load. Naming: pass, dtype and head dim (b64 =
 // bf16 d = 64, b128, f64 = fp32 d = 64), c / n = causal / not, then the
 // variant (waves per SIMD w*, query tiles per wave q*, d = computes Delta,
-// pg = K/V through a block table, g4 = 4 waves per work-group, sp = one split of the keys, p2 = a softmax
+// pg = K/V through a block table, g8 = 8 waves per work-group, sp = one split of the keys, p2 = a softmax
 // scale that is a power of two).
 #pragma once
 
@@ -16,9 +16,9 @@
     X(mxfa_fwd_b64_c_w3_q2) X(mxfa_fwd_b64_c_w2_q2) X(mxfa_fwd_b64_c_w3_q1)                   \
     X(mxfa_fwd_b64_n_w2_q2) X(mxfa_fwd_b64_n_w3_q1)                                           \
     X(mxfa_fwd_b128_c_w2_q2) X(mxfa_fwd_b128_c_w2_q1) X(mxfa_fwd_b128_n_w2_q2)                \
-    X(mxfa_fwd_f64_c) X(mxfa_fwd_f64_n) X(mxfa_fwd_f64_c_g4) X(mxfa_fwd_f64_n_g4)              \
+    X(mxfa_fwd_f64_c) X(mxfa_fwd_f64_n) X(mxfa_fwd_f64_c_g8) X(mxfa_fwd_f64_n_g8)              \
     X(mxfa_fwd_b64_c_w2_q2_pg) X(mxfa_fwd_b64_c_w3_q1_pg) X(mxfa_fwd_b128_c_w2_q1_pg)          \
-    X(mxfa_fwd_f64_c_pg)                                                                      \
+    X(mxfa_fwd_f64_c_pg) X(mxfa_fwd_f64_c_pg_g8)                                              \
     X(mxfa_fwd_b64_c_w3_q1_sp) X(mxfa_fwd_b128_c_w2_q1_sp) X(mxfa_fwd_f64_c_sp)                \
     X(mxfa_fwd_b64_c_w3_q1_pg_sp) X(mxfa_fwd_b128_c_w2_q1_pg_sp) X(mxfa_fwd_f64_c_pg_sp)       \
     X(mxfa_fwd_merge8_b64) X(mxfa_fwd_merge8_b128) X(mxfa_fwd_merge8_f64)                     \
