@@ -174,6 +174,28 @@ def load_library(path: str | None = None):
     return lib
 
 
+_native = None
+
+
+def _calls():
+    """The call path in C++ (csrc/binding.cpp), bound to the loaded libmxfa: its
+    functions take plain GPU tensors on torch's current stream and return
+    NotImplemented for every other call, which the Python below then takes."""
+    global _native
+    if _native is None:
+        lib = load_library()
+        try:
+            from . import _binding as ext
+        except ImportError as e:
+            raise ImportError(f"{os.path.join(_HERE, '_binding.so')} cannot be loaded ({e}): build it with "
+                              "`make -C mx230_amd/csrc` (or __graft_entry__.build())") from e
+        ext.bind(*(ctypes.cast(getattr(lib, f), ctypes.c_void_p).value for f in (
+            "mxfa_run_flash_lse", "mxfa_run_bwd_ws", "mxfa_bwd_workspace_bytes", "mxfa_run_prefill",
+            "mxfa_run_prefill_ws", "mxfa_run_prefill_paged", "mxfa_run_prefill_paged_ws")))
+        _native = ext
+    return _native
+
+
 def _check(func: str, rc: int):
     if rc != 0:
         raise MxfaError(func, rc, load_library().mxfa_strerror(rc).decode())
@@ -597,6 +619,10 @@ def run_prefill(q, kcache, vcache, out, pos0: int, n_head: int, n_kv_head: int, 
     >= n_kv_head*head_dim], same row stride, rows 0..pos0 + n_tok - 1 filled;
     out: [n_tok, >= n_head*head_dim]. All bf16, or fp32 with head_dim 64."""
     torch = _torch()
+    if stream is None:
+        rc = _calls().prefill(q, kcache, vcache, out, None, 0, pos0, n_head, n_kv_head, head_dim, scale, False, None)
+        if rc is not NotImplemented:
+            return _check("mxfa_run_prefill", rc)
     if q.dtype not in (torch.bfloat16, torch.float32):
         raise ValueError(f"q: dtype {q.dtype}; bf16 or float32 expected")
     n_tok = q.shape[0] if q.dim() == 2 else -1
@@ -629,6 +655,12 @@ def run_prefill_paged(q, kcache, vcache, out, block_table, block_size: int, pos0
     does (workspace as there, allocated here when None and returned); its
     outputs equal run_prefill_split's over the gathered cache bit for bit."""
     torch = _torch()
+    if stream is None and (workspace is not None or not split):
+        rc = _calls().prefill(q, kcache, vcache, out, block_table, block_size, pos0, n_head, n_kv_head, head_dim,
+                                scale, split, workspace)
+        if rc is not NotImplemented:
+            _check("mxfa_run_prefill_paged_ws" if split else "mxfa_run_prefill_paged", rc)
+            return workspace if split else None
     if q.dtype not in (torch.bfloat16, torch.float32):
         raise ValueError(f"q: dtype {q.dtype}; bf16 or float32 expected")
     n_tok = q.shape[0] if q.dim() == 2 else -1
@@ -692,6 +724,12 @@ def run_prefill_split(q, kcache, vcache, out, pos0: int, n_head: int, n_kv_head:
     mxfa_prefill_workspace_bytes reports (allocated here when None). Results
     equal run_prefill's to fp32 rounding, not bitwise."""
     torch = _torch()
+    if stream is None and workspace is not None:
+        rc = _calls().prefill(q, kcache, vcache, out, None, 0, pos0, n_head, n_kv_head, head_dim, scale, True,
+                                workspace)
+        if rc is not NotImplemented:
+            _check("mxfa_run_prefill_ws", rc)
+            return workspace
     if q.dtype not in (torch.bfloat16, torch.float32):
         raise ValueError(f"q: dtype {q.dtype}; bf16 or float32 expected")
     n_tok = q.shape[0] if q.dim() == 2 else -1
@@ -717,6 +755,12 @@ def run_prefill_split(q, kcache, vcache, out, pos0: int, n_head: int, n_kv_head:
 def attention_fwd(q, k, v, causal: bool, scale: float = 0.0, stream=None):
     """Allocates O and LSE and runs the forward; returns (O, LSE)."""
     torch = _torch()
+    if stream is None:
+        r = _calls().attention_fwd(q, k, v, causal, scale)
+        if isinstance(r, tuple):
+            return r
+        if r is not NotImplemented:
+            _check("mxfa_run_flash_lse", r)
     sh = shape_of(q, k, causal, scale)
     o = torch.empty_like(q)
     lse = torch.empty((sh.B, sh.Hq, sh.N), dtype=torch.float32, device=q.device)
@@ -729,6 +773,12 @@ def attention_bwd(q, k, v, o, lse, do, causal: bool, scale: float = 0.0, stream=
     workspace) and runs the backward (run_bwd_ws: Delta folded into the dQ
     pass); returns (dQ, dK, dV)."""
     torch = _torch()
+    if stream is None:
+        r = _calls().attention_bwd(q, k, v, o, lse, do, causal, scale)
+        if isinstance(r, tuple):
+            return r
+        if r is not NotImplemented:
+            _check("mxfa_run_bwd_ws", r)
     sh = shape_of(q, k, causal, scale)
     delta = torch.empty((sh.B, sh.Hq, sh.N), dtype=torch.float32, device=q.device)
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
