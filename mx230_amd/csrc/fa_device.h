@@ -734,13 +734,22 @@ struct RowPlan {
 
 // stage_rows with a RowPlan: rows >= nvalid re-read row nvalid - 1, as there.
 // The tile as an LDS address (tile_lds), or as a pointer below.
+// One wave staging a whole tile (NT = 64) loads the even chunks first, then the
+// odd: consecutive loads then read the same 32 rows' next columns, while the
+// rows' lines are in the L1 (one token of 32/8 heads, d = 128, after 65535
+// positions 56 -> 50 us).
+template <int NT, int NK>
+__device__ __forceinline__ constexpr int load_order(int j) {
+    return NT == 64 ? (j < NK / 2 ? 2 * j : 2 * j - NK + 1) : j;
+}
 template <class Pol, int NT = 256>
 __device__ __forceinline__ void stage_rows(uint32_t tile_lds, const typename Pol::T *src, int nvalid,
                                            const RowPlan<Pol, NT> &pl, int wave, int row_stride = Pol::D) {
     const uint32_t base = tile_lds + wave * 64 * 16;
     const uint32_t rs_bytes = (uint32_t)row_stride * sizeof(typename Pol::T);
 #pragma unroll
-    for (int k = 0; k < RowPlan<Pol, NT>::NK; ++k) {
+    for (int j = 0; j < RowPlan<Pol, NT>::NK; ++j) {
+        const int k = load_order<NT, RowPlan<Pol, NT>::NK>(j);
         const uint32_t grow = (uint32_t)min((int)(pl.rc[k] & 255u), nvalid - 1);
         lds_dma16_s(base + k * NT * 16, src, grow * rs_bytes + (pl.rc[k] >> 8));
     }
@@ -802,6 +811,19 @@ struct PagedRows {
             lds_dma16(bv + k * NT * 16, V + off);
         }
     }
+    // the same rows of one tensor
+    __device__ __forceinline__ void stage_one(typename Pol::T *tile, const typename Pol::T *X, int k0, int N, int shift,
+                                              const RowPlan<Pol, NT> &pl, int wave, int row_stride) const {
+        const uint32_t base = lds_addr(tile) + wave * 64 * 16;
+        const int mask = (1 << shift) - 1;
+#pragma unroll
+        for (int j = 0; j < NK; ++j) {
+            const int k = load_order<NT, NK>(j);
+            const int t = min(k0 + (int)(pl.rc[k] & 255u), N - 1);
+            lds_dma16(base + k * NT * 16, X + ((((size_t)blk[k] << shift) + (size_t)(t & mask)) * (size_t)row_stride +
+                                               (pl.rc[k] >> 8) / sizeof(typename Pol::T)));
+        }
+    }
 };
 
 // Read by lanes past the end of a staged vector (see stage_vec64). Device
@@ -826,6 +848,9 @@ __device__ __forceinline__ void stage_vec64(float *dst, const float *src, int nv
 // Waits for this wave's outstanding global->LDS loads (the caller then
 // barriers so every wave's loads are visible).
 __device__ __forceinline__ void wait_stage() { __builtin_amdgcn_s_waitcnt(0); }
+
+// Waits for this wave's LDS operations.
+__device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
 // Workgroup barrier that waits only for this wave's LDS operations.
 // __syncthreads() also waits for every outstanding vector-memory operation
@@ -852,6 +877,13 @@ template <int VM>
 __device__ __forceinline__ void wait_vmcnt() {
     static_assert(VM >= 0 && VM < 64, "vmcnt is 6 bits");
     __builtin_amdgcn_s_waitcnt((VM & 15) | ((VM >> 4) << 14) | (7 << 4) | (15 << 8));
+}
+
+// The same, and no memory access moves across it: for global->LDS loads that no
+// barrier follows (a wave's own tile).
+template <int VM>
+__device__ __forceinline__ void wait_loads() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(VM) : "memory");
 }
 
 // Global->LDS loads one thread of an NT-thread workgroup issues for one

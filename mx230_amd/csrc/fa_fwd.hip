@@ -46,11 +46,18 @@ __device__ __forceinline__ constexpr int fwd_mask_offset(int blk, int t, int g, 
 // O^T += V^T P^T. PRIO: the matrix products run at raised wave priority.
 // qpos0: position of the wave's first query row; Nk: key rows. EMPTY_ROWS:
 // rows may have every key of the stage masked (a key split's first stage).
-template <class Pol, int QT, bool CAUSAL, bool MASK, bool PRIO = false, bool EMPTY_ROWS = false>
+// after_k runs once K has been read, before_v before V is (fwd_few_entry's
+// loads and waits).
+struct FwdNothing {
+    __device__ __forceinline__ void operator()() const {}
+};
+template <class Pol, int QT, bool CAUSAL, bool MASK, bool PRIO = false, bool EMPTY_ROWS = false,
+          class AfterK = FwdNothing, class BeforeV = FwdNothing>
 __device__ __forceinline__ void fwd_stage(f32x4 (&acc)[Pol::D / 16][QT], float (&m)[QT], float (&lsum)[QT],
                                           const typename Pol::Frag (&qf)[QT][Pol::NC],
                                           const typename Pol::T *sk, const typename Pol::T *sv, int k0, int qpos0,
-                                          int Nk, int g, int l16, float xmul) {
+                                          int Nk, int g, int l16, float xmul, AfterK after_k = {},
+                                          BeforeV before_v = {}) {
     using Frag = typename Pol::Frag;
     constexpr int NC = Pol::NC, XT = Pol::D / 16;
     f32x4 s[2][2][QT];  // [block][t][qt]
@@ -71,6 +78,7 @@ __device__ __forceinline__ void fwd_stage(f32x4 (&acc)[Pol::D / 16][QT], float (
         }
     }
     wave_priority<PRIO>(0);
+    after_k();
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
         const int lim = fwd_mask_limit<Pol, CAUSAL>(qpos0 + 16 * qt + l16, k0, Nk, g);
@@ -112,6 +120,7 @@ __device__ __forceinline__ void fwd_stage(f32x4 (&acc)[Pol::D / 16][QT], float (
         }
         lsum[qt] = ls;
     }
+    before_v();
     wave_priority<PRIO>(1);
 #pragma unroll
     for (int blk = 0; blk < 2; ++blk) {
@@ -457,6 +466,133 @@ __device__ __forceinline__ void fwd_entry(const Params &p) {
     wg_time_after_stores();
 }
 
+// The forward of a few query rows (at most 16 per head: a token's GQA group, or
+// a handful of tokens) over a KV cache, bf16. All NW waves hold the same rows;
+// each takes 64-key stages of its own (the work-group's stages [s_lo, s_hi),
+// every NW-th), staged into its own LDS tiles with no barrier between waves, and
+// the waves' running maxima, sums and O are merged through LDS at the end.
+//
+// Bound: the loads. A work-group has NW x 64 keys of K and V in flight (128 KB,
+// one work-group per CU), where the 64-query form holds one stage ahead and
+// leaves three of its four waves without rows. Kernel-trace medians of one
+// token with its keys split, us: 14/2 heads after 65535 20.2 -> 9.0 (3.7 TB/s;
+// 128 splits instead of 32), 32/4 heads after 4095, paged, 5.0 -> 4.6.
+constexpr int kFewRows = 16;
+
+template <class Pol, int NW>
+union FwdFewSmem {
+    struct {
+        typename Pol::T k[NW][Pol::ROWS * Pol::D], v[NW][Pol::ROWS * Pol::D];
+    } t;
+    struct {
+        float acc[NW][kFewRows][Pol::D + 4];
+        float ml[NW][kFewRows][2];
+    } merge;
+};
+
+template <class Pol, int NW, bool PAGED, bool SPLIT>
+__device__ __forceinline__ void fwd_few_entry(const Params &p) {
+    using T = typename Pol::T;
+    constexpr int D = Pol::D, XT = D / 16, BK = Pol::ROWS;
+    __shared__ __attribute__((aligned(16))) FwdFewSmem<Pol, NW> sm;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = lane >> 4, l16 = lane & 15;
+    const int N = p.N, Nk = p.Nk, bh = blockIdx.x;
+    const int b = bh / p.Hq, h = bh % p.Hq, kvh = h / p.group;
+    const size_t kvoff = b * p.kv_bs + kvh * p.kv_hs;
+    const T *K = static_cast<const T *>(p.k) + kvoff, *V = static_cast<const T *>(p.v) + kvoff;
+    T *sk = sm.t.k[wave], *sv = sm.t.v[wave];
+    wg_time(0);
+    const int nsteps = (min(Nk, p.pos0 + N) + BK - 1) / BK;
+    const int s_lo = SPLIT ? (int)((long long)blockIdx.z * nsteps / gridDim.z) : 0;
+    const int s_hi = SPLIT ? (int)((long long)(blockIdx.z + 1) * nsteps / gridDim.z) : nsteps;
+    wg_info(2, 0, s_hi - s_lo);
+
+    const RowPlan<Pol, 64> plan(lane);
+    PagedRows<Pol, 64> paged;
+    constexpr int NL = RowPlan<Pol, 64>::NK;  // loads of a tile
+    auto load = [&](T *tile, const T *base, int st) __attribute__((always_inline)) {
+        if constexpr (PAGED) {
+            paged.stage_one(tile, base, st * BK, Nk, p.bs_shift, plan, 0, p.kv_rs);
+        } else {
+            stage_rows<Pol, 64>(tile, base + (size_t)(st * BK) * p.kv_rs, Nk - st * BK, plan, 0, p.kv_rs);
+        }
+    };
+    auto fetch = [&](int st) __attribute__((always_inline)) {
+        if constexpr (PAGED) paged.fetch(p.block_table, p.bs_shift, st * BK, Nk, plan);
+    };
+    int st = s_lo + wave;
+    if (st < s_hi) {
+        fetch(st);
+        load(sk, K, st);
+        load(sv, V, st);
+    }
+    typename Pol::Frag qf[1][Pol::NC];
+    Pol::gmem_row_frags(qf[0], static_cast<const T *>(p.q) + b * p.q_bs + h * p.q_hs, l16, N, p.q_rs, g);
+    f32x4 acc[XT][1];
+#pragma unroll
+    for (int xt = 0; xt < XT; ++xt) acc[xt][0] = zero4();
+    float m[1] = {-INFINITY}, lsum[1] = {0.f};
+    // The wave's next stage: its K goes out once this one's K has been read, its
+    // V once this one's V has, so one tile is in flight at any time. At least
+    // NL loads follow K's when it is waited for (this stage's V), and V's (the
+    // next K): vmcnt counts in order.
+    for (; st < s_hi; st += NW) {
+        const bool more = st + NW < s_hi;
+        if (more) fetch(st + NW);
+        wait_loads<NL>();
+        fwd_stage<Pol, 1, true, true, false, true>(
+            acc, m, lsum, qf, sk, sv, st * BK, p.pos0, Nk, g, l16, p.scale_log2,
+            [&]() __attribute__((always_inline)) {
+                wait_lds();
+                if (more) load(sk, K, st + NW);
+            },
+            [&]() __attribute__((always_inline)) {
+                if (more) {
+                    wait_loads<NL>();
+                } else {
+                    wait_loads<0>();
+                }
+            });
+        wait_lds();
+        if (more) load(sv, V, st + NW);
+    }
+    const float lw = xg_sum(lsum[0]);
+    __syncthreads();  // every wave is done with the tiles
+    wg_time(2);
+#pragma unroll
+    for (int xt = 0; xt < XT; ++xt)
+        *reinterpret_cast<f32x4 *>(&sm.merge.acc[wave][l16][16 * xt + 4 * g]) = acc[xt][0];
+    if (g == 0) *reinterpret_cast<float2 *>(sm.merge.ml[wave][l16]) = make_float2(m[0], lw);
+    __syncthreads();
+    for (int i = tid; i < N * (D / 4); i += 64 * NW) {
+        const int r = i / (D / 4), c = 4 * (i % (D / 4));
+        float M = -INFINITY, L = 0.f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) M = fmaxf(M, sm.merge.ml[w][r][0]);
+        const float mref = M == -INFINITY ? 0.f : M;  // a split with no key of the row: weight 0
+        f32x4 o = zero4();
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            const float x = fast_exp2(sm.merge.ml[w][r][0] - mref);
+            L += x * sm.merge.ml[w][r][1];
+            o += *reinterpret_cast<const f32x4 *>(&sm.merge.acc[w][r][c]) * x;
+        }
+        if constexpr (SPLIT) {
+            const size_t rows = (size_t)gridDim.z * p.B * p.Hq * N;
+            const size_t r0 = ((size_t)blockIdx.z * p.B * p.Hq + bh) * N + r;
+            store4<float>(p.fwd_part + r0 * D + c, o, 1.0f);
+            if (c == 0) *reinterpret_cast<float2 *>(p.fwd_part + rows * D + 2 * r0) = make_float2(M, L);
+        } else {
+            T *O = static_cast<T *>(p.o) + b * p.o_bs + h * p.o_hs + (size_t)r * p.o_rs;
+            store4<T>(O + c, o, 1.0f / L);
+            if (p.lse != nullptr && c == 0) p.lse[(size_t)bh * N + r] = (M + fast_log2(L)) * kLn2;
+        }
+    }
+    wg_time_after_stores();
+}
+
 // The fp32 forward (d = 64) with its products in bf16 parts (Split3): NW waves
 // of 16 queries, 64 keys per stage. K and V pass through registers, loaded one
 // stage ahead, and are split once per work-group into one 48 KB LDS buffer;
@@ -719,15 +855,19 @@ __device__ __forceinline__ void fwd_split_entry(const Params &p) {
     wg_time_after_stores();
 }
 
-// Adds the S key splits of a split forward (fwd_entry<..., SPLIT>), one
-// thread per four elements of a query row: with M the largest of the splits'
-// running maxima (log2 units), O = sum_s 2^(m_s - M) O_s / sum_s 2^(m_s - M)
-// l_s, in split order, written as the forward writes O. A split that holds
-// no key of the row has m = -inf and weight 0. Every load is issued before
-// the first is used (the loops unrolled to MAXS >= S), so a call costs one
-// memory latency rather than one per split; MAXS = 8 keeps the registers of
-// the common case low (the 32-split form takes 205 VGPRs).
-constexpr int kFwdMaxSplits = 32;
+// Adds the S key splits of a split forward (fwd_entry<..., SPLIT>): with M the
+// largest of the splits' running maxima (log2 units), O = sum_s 2^(m_s - M)
+// O_s / sum_s 2^(m_s - M) l_s, written as the forward writes O. A split that
+// holds no key of the row has m = -inf and weight 0. Up to kMergeThread splits
+// (many rows then): one thread per four elements of a row, every split's loads
+// issued before the first is used, so a call costs one memory latency. More
+// splits (few rows): a work-group per row, its groups of threads over the
+// (fwd_merge_row_body): with a thread per four elements one token's 32 rows
+// are two work-groups, each reading 131 KB (32 splits 4.7 -> 3.1 us; the
+// 128 splits of 14 rows 3.6).
+constexpr int kFwdMaxSplits = 32;   // of 64-query work-groups
+constexpr int kFewMaxSplits = 128;  // of fwd_few_entry's
+constexpr int kMergeThread = 8;
 
 template <class T, int D, int MAXS>
 __device__ __forceinline__ void fwd_merge_body(const Params &p, int S) {
@@ -763,6 +903,68 @@ __device__ __forceinline__ void fwd_merge_body(const Params &p, int S) {
             o[2] += w * a[sp].z;
             o[3] += w * a[sp].w;
         }
+    }
+    const int bh = (int)(r / p.N), qi = (int)(r % p.N);
+    const int b = bh / p.Hq, h = bh % p.Hq;
+    T *O = static_cast<T *>(p.o) + b * p.o_bs + h * p.o_hs + (size_t)qi * p.o_rs + 4 * c;
+    store4<T>(O, o, 1.0f / L);
+    if (p.lse != nullptr && c == 0) p.lse[r] = (M + fast_log2(L)) * kLn2;
+}
+
+template <class T, int D, int MAXS>
+__device__ __forceinline__ void fwd_merge_row_body(const Params &p, int S) {
+    constexpr int NT = 8 * MAXS, NW = NT / 64;
+    constexpr int C = D / 4, G = NT / C, PER = MAXS / G;  // threads per row of O, groups of splits, splits per group
+    static_assert(PER * G == MAXS && 64 % C == 0, "whole groups, and whole waves of them");
+    __shared__ float sm[NW], sl[NW];
+    __shared__ __attribute__((aligned(16))) f32x4 so[NW][C];
+    const size_t rows = (size_t)p.B * p.Hq * p.N, r = blockIdx.x;
+    const int tid = threadIdx.x, wave = tid / 64, c = tid % C, grp = tid / C;
+    const float2 *ml = reinterpret_cast<const float2 *>(p.fwd_part + (size_t)S * rows * D);
+    float2 v[PER];
+    f32x4 a[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int sp = grp + G * i;
+        v[i] = make_float2(-INFINITY, 0.f);
+        a[i] = zero4();
+        if (sp < S) {
+            v[i] = ml[sp * rows + r];
+            a[i] = *reinterpret_cast<const f32x4 *>(p.fwd_part + (sp * rows + r) * D + 4 * c);
+        }
+    }
+    float M = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) M = fmaxf(M, v[i].x);
+#pragma unroll
+    for (int k = 32; k >= C; k >>= 1) M = fmaxf(M, __shfl_xor(M, k, 64));
+    if (tid % 64 == 0) sm[wave] = M;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < NW; ++w) M = fmaxf(M, sm[w]);  // finite: the split of key 0
+    float L = 0.f;
+    f32x4 o = zero4();
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const float w = fast_exp2(v[i].x - M);
+        L += w * v[i].y;
+        o += a[i] * w;
+    }
+    // the wave's groups, then the waves
+#pragma unroll
+    for (int k = 32; k >= C; k >>= 1) {
+        L += __shfl_xor(L, k, 64);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] += __shfl_xor(o[e], k, 64);
+    }
+    if (tid % 64 < C) so[wave][c] = o;
+    if (tid % 64 == 0) sl[wave] = L;
+    __syncthreads();
+    if (tid >= C) return;
+#pragma unroll
+    for (int w = 1; w < NW; ++w) {
+        o += so[w][c];
+        L += sl[w];
     }
     const int bh = (int)(r / p.N), qi = (int)(r % p.N);
     const int b = bh / p.Hq, h = bh % p.Hq;
@@ -818,17 +1020,37 @@ MXFA_FWD_SP(mxfa_fwd_b128_c_w2_q1_pg_sp, PolBF16<128>, 2, true)
     extern "C" __global__ __launch_bounds__(256) void NAME(Params p, int splits) {                     \
         fwd_merge_body<T, D, MAXS>(p, splits);                                                         \
     }
-MXFA_FWD_MERGE(mxfa_fwd_merge8_b64, u16, 64, 8)
-MXFA_FWD_MERGE(mxfa_fwd_merge8_b128, u16, 128, 8)
-MXFA_FWD_MERGE(mxfa_fwd_merge8_f64, float, 64, 8)
-MXFA_FWD_MERGE(mxfa_fwd_merge32_b64, u16, 64, kFwdMaxSplits)
-MXFA_FWD_MERGE(mxfa_fwd_merge32_b128, u16, 128, kFwdMaxSplits)
-MXFA_FWD_MERGE(mxfa_fwd_merge32_f64, float, 64, kFwdMaxSplits)
+MXFA_FWD_MERGE(mxfa_fwd_merge8_b64, u16, 64, kMergeThread)
+MXFA_FWD_MERGE(mxfa_fwd_merge8_b128, u16, 128, kMergeThread)
+MXFA_FWD_MERGE(mxfa_fwd_merge8_f64, float, 64, kMergeThread)
+#define MXFA_FWD_MERGE_ROW(NAME, T, D, MAXS)                                                           \
+    extern "C" __global__ __launch_bounds__(8 * MAXS) void NAME(Params p, int splits) {                \
+        fwd_merge_row_body<T, D, MAXS>(p, splits);                                                     \
+    }
+MXFA_FWD_MERGE_ROW(mxfa_fwd_merge32_b64, u16, 64, kFwdMaxSplits)
+MXFA_FWD_MERGE_ROW(mxfa_fwd_merge32_b128, u16, 128, kFwdMaxSplits)
+MXFA_FWD_MERGE_ROW(mxfa_fwd_merge32_f64, float, 64, kFwdMaxSplits)
+MXFA_FWD_MERGE_ROW(mxfa_fwd_merge128_b64, u16, 64, kFewMaxSplits)
+MXFA_FWD_MERGE_ROW(mxfa_fwd_merge128_b128, u16, 128, kFewMaxSplits)
+#define MXFA_FWD_FEW(NAME, D, NW, PG, SP)                                                              \
+    extern "C" __global__ __launch_bounds__(64 * NW) void NAME(Params p) {                             \
+        fwd_few_entry<PolBF16<D>, NW, PG, SP>(p);                                                      \
+    }
+MXFA_FWD_FEW(mxfa_fwd_b64_few, 64, 8, false, false)
+MXFA_FWD_FEW(mxfa_fwd_b64_few_pg, 64, 8, true, false)
+MXFA_FWD_FEW(mxfa_fwd_b64_few_sp, 64, 8, false, true)
+MXFA_FWD_FEW(mxfa_fwd_b64_few_pg_sp, 64, 8, true, true)
+MXFA_FWD_FEW(mxfa_fwd_b128_few, 128, 4, false, false)
+MXFA_FWD_FEW(mxfa_fwd_b128_few_pg, 128, 4, true, false)
+MXFA_FWD_FEW(mxfa_fwd_b128_few_sp, 128, 4, false, true)
+MXFA_FWD_FEW(mxfa_fwd_b128_few_pg_sp, 128, 4, true, true)
 #undef MXFA_FWD
 #undef MXFA_FWD_F
 #undef MXFA_FWD_PG
 #undef MXFA_FWD_SP
 #undef MXFA_FWD_MERGE
+#undef MXFA_FWD_MERGE_ROW
+#undef MXFA_FWD_FEW
 #endif
 
 // The kernel of (policy, causal) compiled for `wps` waves per SIMD with `qt`
@@ -905,6 +1127,29 @@ static hipError_t launch_fwd_f32(Params p, int causal, hipStream_t stream) {
     return launch_kernel(id, grid, dim3(64 * nw), args, stream);
 }
 
+// Few query rows of a prefill: fwd_few_entry, unsplit at any number of keys (one
+// token, us a call: 8/1 heads d = 128 after 2000 positions 27.2 -> 17.1, 14/2
+// heads after 65535 555 -> 370, 32/32 heads after 8191 paged 78 -> 70), and
+// split where the 256 work-groups that fit at once (8 waves; d = 128: 4) leave
+// each wave at most two stages. Beyond that the 64-query form's work-groups,
+// whose waves load each tile together, read faster: 14/2 heads after 65535
+// 24.6 -> 13.1, 8/8 after 20000 17.4 -> 13.5, but 32/8 after 65535 26.5
+// against 30.9, and d = 128 45 against 50.
+static bool fwd_few(const Params &p, int dtype_bf16) { return dtype_bf16 && p.prefill != 0 && p.N <= kFewRows; }
+static bool fwd_few_split(const Params &p, int dtype_bf16, int d) {
+    const long long stages = (std::min(p.Nk, p.pos0 + p.N) + 63) / 64;
+    return fwd_few(p, dtype_bf16) && (long long)p.B * p.Hq * stages <= 2 * 256 * (d == 128 ? 4 : 8);
+}
+
+static hipError_t launch_fwd_few(const Params &p, int d, int splits, hipStream_t stream) {
+    const bool pg = p.block_table != nullptr, sp = splits > 1;
+    static constexpr KernelId ids[2][2][2] = {
+        {{k_mxfa_fwd_b64_few, k_mxfa_fwd_b64_few_sp}, {k_mxfa_fwd_b64_few_pg, k_mxfa_fwd_b64_few_pg_sp}},
+        {{k_mxfa_fwd_b128_few, k_mxfa_fwd_b128_few_sp}, {k_mxfa_fwd_b128_few_pg, k_mxfa_fwd_b128_few_pg_sp}}};
+    void *args[] = {const_cast<Params *>(&p)};
+    return launch_kernel(ids[d == 128][pg][sp], dim3(p.B * p.Hq, 1, splits), dim3(d == 128 ? 256 : 512), args, stream);
+}
+
 // Splits of the prefill's keys: none (1) when the 64-query work-groups
 // already fill the resident slots (256 CUs x waves per SIMD) halfway, or when
 // the heaviest query block has under 16 key stages (bf16; 8 for fp32), where
@@ -920,7 +1165,15 @@ int fwd_splits(const Params &p, int dtype_bf16, int d) {
     if (stages < (dtype_bf16 ? 16 : 8)) return 1;
     long long s = (slots + wgs - 1) / wgs;
     s = std::min(s, std::max(1LL, stages / 2));
+    // fwd_few_entry: one work-group to a CU, in one round
+    if (fwd_few_split(p, dtype_bf16, d)) return (int)std::min({s, (long long)kFewMaxSplits, std::max(1LL, 256 / wgs)});
     return (int)std::min(s, (long long)kFwdMaxSplits);
+}
+
+int fwd_splits_in(const Params &p, int d, int splits, size_t bytes) {
+    const size_t one = (size_t)p.B * p.Hq * p.N * (size_t)(d + 2) * sizeof(float);
+    if (bytes / one >= (size_t)splits) return splits;
+    return bytes / one >= (size_t)kFwdMaxSplits ? (int)(bytes / one) : 0;
 }
 
 size_t fwd_split_workspace_bytes(const Params &p, int d, int splits) {
@@ -929,28 +1182,33 @@ size_t fwd_split_workspace_bytes(const Params &p, int d, int splits) {
 }
 
 hipError_t launch_fwd_split(const Params &p, int dtype_bf16, int d, int splits, hipStream_t stream) {
-    if (p.fwd_part == nullptr || splits < 2 || splits > kFwdMaxSplits) return hipErrorInvalidValue;
-    const bool pg = p.block_table != nullptr;
+    const bool few = fwd_few_split(p, dtype_bf16, d), pg = p.block_table != nullptr;
+    if (p.fwd_part == nullptr || splits < 2 || splits > (few ? kFewMaxSplits : kFwdMaxSplits)) return hipErrorInvalidValue;
     const KernelId kf =
         dtype_bf16 ? (d == 64 ? (pg ? k_mxfa_fwd_b64_c_w3_q1_pg_sp : k_mxfa_fwd_b64_c_w3_q1_sp)
                               : (pg ? k_mxfa_fwd_b128_c_w2_q1_pg_sp : k_mxfa_fwd_b128_c_w2_q1_sp))
                    : (pg ? k_mxfa_fwd_f64_c_pg_sp : k_mxfa_fwd_f64_c_sp);
-    const bool m8 = splits <= 8;
-    const KernelId km = dtype_bf16 ? (d == 64 ? (m8 ? k_mxfa_fwd_merge8_b64 : k_mxfa_fwd_merge32_b64)
-                                              : (m8 ? k_mxfa_fwd_merge8_b128 : k_mxfa_fwd_merge32_b128))
-                                   : (m8 ? k_mxfa_fwd_merge8_f64 : k_mxfa_fwd_merge32_f64);
+    const int mi = splits <= kMergeThread ? 0 : splits <= kFwdMaxSplits ? 1 : 2;  // 2: few rows, bf16
+    static constexpr KernelId merge[3][3] = {
+        {k_mxfa_fwd_merge8_b64, k_mxfa_fwd_merge32_b64, k_mxfa_fwd_merge128_b64},
+        {k_mxfa_fwd_merge8_b128, k_mxfa_fwd_merge32_b128, k_mxfa_fwd_merge128_b128},
+        {k_mxfa_fwd_merge8_f64, k_mxfa_fwd_merge32_f64, k_mxfa_fwd_merge32_f64}};
+    const KernelId km = merge[!dtype_bf16 ? 2 : d == 128 ? 1 : 0][mi];
     Params q = p;
     void *args[] = {&q};
-    hipError_t e = launch_kernel(kf, dim3(p.B * p.Hq, (p.N + 63) / 64, splits), dim3(256), args, stream);
+    hipError_t e = few ? launch_fwd_few(p, d, splits, stream)
+                       : launch_kernel(kf, dim3(p.B * p.Hq, (p.N + 63) / 64, splits), dim3(256), args, stream);
     if (e != hipSuccess) return e;
-    const size_t n = (size_t)p.B * p.Hq * p.N * (d / 4);
+    const size_t rows = (size_t)p.B * p.Hq * p.N;
     int s = splits;
     void *margs[] = {&q, &s};
-    return launch_kernel(km, dim3((unsigned)((n + 255) / 256)), dim3(256), margs, stream);
+    const unsigned groups = (unsigned)(mi == 0 ? (rows * (d / 4) + 255) / 256 : rows);
+    return launch_kernel(km, dim3(groups), dim3(mi == 2 ? 8 * kFewMaxSplits : 256), margs, stream);
 }
 
 hipError_t launch_fwd(const Params &p, int dtype_bf16, int d, int causal, hipStream_t stream) {
     if (p.block_table != nullptr && !causal) return hipErrorInvalidValue;  // paged kernels are causal
+    if (causal && fwd_few(p, dtype_bf16)) return launch_fwd_few(p, d, 1, stream);
     if (!dtype_bf16) return d == 64 ? launch_fwd_f32(p, causal, stream) : hipErrorInvalidValue;
     if (d == 64) return causal ? launch_fwd_t<PolBF16<64>, true>(p, stream) : launch_fwd_t<PolBF16<64>, false>(p, stream);
     if (d == 128)

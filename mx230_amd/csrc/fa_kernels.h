@@ -7,7 +7,7 @@
 // the code object fails that load. Naming: pass, dtype and head dim (b64 =
 // bf16 d = 64, b128, f64 = fp32 d = 64), c / n = causal / not, then the
 // variant (waves per SIMD w*, query tiles per wave q*, d = computes Delta,
-// pg = K/V through a block table, g8 = 8 waves per work-group, sp = one split of the keys, p2 = a softmax
+// pg = K/V through a block table, g8 = 8 waves per work-group, few = at most 16 query rows, sp = one split of the keys, p2 = a softmax
 // scale that is a power of two).
 #pragma once
 
@@ -23,6 +23,9 @@
     X(mxfa_fwd_b64_c_w3_q1_pg_sp) X(mxfa_fwd_b128_c_w2_q1_pg_sp) X(mxfa_fwd_f64_c_pg_sp)       \
     X(mxfa_fwd_merge8_b64) X(mxfa_fwd_merge8_b128) X(mxfa_fwd_merge8_f64)                     \
     X(mxfa_fwd_merge32_b64) X(mxfa_fwd_merge32_b128) X(mxfa_fwd_merge32_f64)                  \
+    X(mxfa_fwd_merge128_b64) X(mxfa_fwd_merge128_b128)                                        \
+    X(mxfa_fwd_b64_few) X(mxfa_fwd_b64_few_pg) X(mxfa_fwd_b64_few_sp) X(mxfa_fwd_b64_few_pg_sp) \
+    X(mxfa_fwd_b128_few) X(mxfa_fwd_b128_few_pg) X(mxfa_fwd_b128_few_sp) X(mxfa_fwd_b128_few_pg_sp) \
     /* backward (fa_bwd.hip) */                                                               \
     X(mxfa_preprocess_b64) X(mxfa_preprocess_b128) X(mxfa_preprocess_f64)                     \
     X(mxfa_dq_b64_c) X(mxfa_dq_b64_c_d) X(mxfa_dq_b64_n) X(mxfa_dq_b64_n_d)                   \

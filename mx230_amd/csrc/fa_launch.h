@@ -46,9 +46,12 @@ void cu_balance(Params *p, KernelId id, long long groups);
 hipError_t launch_fwd(const Params &p, int dtype_bf16, int d, int causal, hipStream_t stream);
 // The causal forward with its keys split over work-groups (grid.z) and a
 // merging launch: the split count for a shape (1: no split pays), the fp32
-// partials it needs in p.fwd_part, and the two launches (2 <= splits <=
-// kFwdMaxSplits = 32; K/V contiguous, or through p.block_table).
+// partials it needs in p.fwd_part, and the two launches (2 <= splits <= 32,
+// or 128 of a few-row shape; K/V contiguous, or through p.block_table).
+// fwd_splits_in: of `splits`, those a workspace of `bytes` holds the partials
+// of, where they are all of them or at least 32 (0: too small).
 int fwd_splits(const Params &p, int dtype_bf16, int d);
+int fwd_splits_in(const Params &p, int d, int splits, size_t bytes);
 size_t fwd_split_workspace_bytes(const Params &p, int d, int splits);
 hipError_t launch_fwd_split(const Params &p, int dtype_bf16, int d, int splits, hipStream_t stream);
 hipError_t launch_preprocess(const Params &p, int dtype_bf16, int d, hipStream_t stream);
