@@ -361,8 +361,9 @@ int mxfa_run_prefill_paged(const mxfa_prefill_shape *shape, const void *q, const
  * device memory (no contents needed; calls that share one race). When that
  * size is 0 the shape needs no split and this is mxfa_run_prefill (workspace
  * may be NULL). A smaller workspace gives MXFA_ERR_WORKSPACE, except that a
- * shape of more than 32 ranges (one token far into a long context) takes one
- * that holds 32 or more of them and uses as many. Results equal
+ * shape that gains from many ranges (one token far into a long context, an
+ * fp32 chunk) takes a smaller one, or none, down to what 64-query blocks take
+ * (at most 32 ranges), and uses as many as it holds. Results equal
  * mxfa_run_prefill's to fp32 rounding of the merge, not bitwise. */
 size_t mxfa_prefill_workspace_bytes(const mxfa_prefill_shape *shape);
 int mxfa_run_prefill_ws(const mxfa_prefill_shape *shape, const void *q, const void *kcache, const void *vcache,

@@ -1001,6 +1001,8 @@ MXFA_FWD_F(mxfa_fwd_f64_c_pg, 4, true, true, false)
 MXFA_FWD_F(mxfa_fwd_f64_c_pg_g8, 8, true, true, false)
 MXFA_FWD_F(mxfa_fwd_f64_c_sp, 4, true, false, true)
 MXFA_FWD_F(mxfa_fwd_f64_c_pg_sp, 4, true, true, true)
+MXFA_FWD_F(mxfa_fwd_f64_c_sp_g8, 8, true, false, true)
+MXFA_FWD_F(mxfa_fwd_f64_c_pg_sp_g8, 8, true, true, true)
 // the prefill over a paged cache (causal, as the prefill always is)
 // (the table entries take registers: the three-wave 128-query d = 64 and the
 // 128-query d = 128 forms would spill in their loops, so paged launches use
@@ -1157,23 +1159,45 @@ static hipError_t launch_fwd_few(const Params &p, int d, int splits, hipStream_t
 // Qwen2.5 heads, 512 tokens at position 0, 8 stages: bf16 19.7 -> 24.6 us
 // with 2 splits, fp32 36.5 -> 32.6 us); else enough to fill them, with at
 // least 2 key stages per split and at most kFwdMaxSplits splits.
-int fwd_splits(const Params &p, int dtype_bf16, int d) {
+static int fwd_splits_64(const Params &p, int dtype_bf16, int d, long long most) {
     const long long wgs = (long long)p.B * p.Hq * ((p.N + 63) / 64);
     const long long slots = 256LL * (dtype_bf16 && d == 64 ? 3 : 2);
     if (2 * wgs >= slots) return 1;
     const long long stages = (std::min(p.Nk, p.pos0 + p.N) + 63) / 64;  // the heaviest block's
     if (stages < (dtype_bf16 ? 16 : 8)) return 1;
-    long long s = (slots + wgs - 1) / wgs;
-    s = std::min(s, std::max(1LL, stages / 2));
-    // fwd_few_entry: one work-group to a CU, in one round
-    if (fwd_few_split(p, dtype_bf16, d)) return (int)std::min({s, (long long)kFewMaxSplits, std::max(1LL, 256 / wgs)});
-    return (int)std::min(s, (long long)kFwdMaxSplits);
+    return (int)std::min({(slots + wgs - 1) / wgs, std::max(1LL, stages / 2), most});
 }
 
-int fwd_splits_in(const Params &p, int d, int splits, size_t bytes) {
+// fp32 chunks of more than 64 rows split over 8-wave work-groups of 128 queries
+// (launch_fwd_f32's reason) where there are stages enough to fill the 512 that
+// fit at once and the blocks alone leave half of them empty: us a call, 14/2
+// heads, 500 tokens after 3584 65 -> 56 (9 splits; 5 of 4-wave work-groups), 70
+// after 8000 40 -> 31; 4/2 heads, 100 after 2000, which cannot fill them,
+// 13.5 against 15.6.
+static bool fwd_f32_wide(const Params &p, int dtype_bf16) {
+    if (dtype_bf16 || p.N <= 64) return false;
+    const long long stages = (std::min(p.Nk, p.pos0 + p.N) + 63) / 64, bh = (long long)p.B * p.Hq;
+    return stages >= 16 && bh * ((p.N + 127) / 128) < 256 &&
+           bh * ((p.N + 63) / 64) * std::min(stages / 2, (long long)kFwdMaxSplits) >= 512;
+}
+
+// The forms that split into one round of the work-groups that fit at once:
+// those, and fwd_few_entry's 256; else fwd_splits_64's.
+int fwd_splits(const Params &p, int dtype_bf16, int d) {
+    const long long stages = (std::min(p.Nk, p.pos0 + p.N) + 63) / 64, bh = (long long)p.B * p.Hq;
+    if (fwd_f32_wide(p, dtype_bf16))
+        return (int)std::min({512 / (bh * ((p.N + 127) / 128)), stages / 2, (long long)kFwdMaxSplits});
+    const bool few = fwd_few_split(p, dtype_bf16, d);
+    const int s = fwd_splits_64(p, dtype_bf16, d, few ? kFewMaxSplits : kFwdMaxSplits);
+    return few ? (int)std::min<long long>(s, std::max(1LL, 256 / bh)) : s;
+}
+
+int fwd_splits_in(const Params &p, int dtype_bf16, int d, size_t bytes) {
+    const int want = fwd_splits(p, dtype_bf16, d), must = fwd_splits_64(p, dtype_bf16, d, kFwdMaxSplits);
     const size_t one = (size_t)p.B * p.Hq * p.N * (size_t)(d + 2) * sizeof(float);
-    if (bytes / one >= (size_t)splits) return splits;
-    return bytes / one >= (size_t)kFwdMaxSplits ? (int)(bytes / one) : 0;
+    const int fit = (int)std::min<size_t>(bytes / one, (size_t)want);
+    if (must <= 1) return std::max(fit, 1);
+    return fit >= std::min(want, must) ? fit : 0;
 }
 
 size_t fwd_split_workspace_bytes(const Params &p, int d, int splits) {
@@ -1184,9 +1208,11 @@ size_t fwd_split_workspace_bytes(const Params &p, int d, int splits) {
 hipError_t launch_fwd_split(const Params &p, int dtype_bf16, int d, int splits, hipStream_t stream) {
     const bool few = fwd_few_split(p, dtype_bf16, d), pg = p.block_table != nullptr;
     if (p.fwd_part == nullptr || splits < 2 || splits > (few ? kFewMaxSplits : kFwdMaxSplits)) return hipErrorInvalidValue;
+    const int nw = fwd_f32_wide(p, dtype_bf16) ? 8 : 4;
     const KernelId kf =
         dtype_bf16 ? (d == 64 ? (pg ? k_mxfa_fwd_b64_c_w3_q1_pg_sp : k_mxfa_fwd_b64_c_w3_q1_sp)
                               : (pg ? k_mxfa_fwd_b128_c_w2_q1_pg_sp : k_mxfa_fwd_b128_c_w2_q1_sp))
+        : nw == 8  ? (pg ? k_mxfa_fwd_f64_c_pg_sp_g8 : k_mxfa_fwd_f64_c_sp_g8)
                    : (pg ? k_mxfa_fwd_f64_c_pg_sp : k_mxfa_fwd_f64_c_sp);
     const int mi = splits <= kMergeThread ? 0 : splits <= kFwdMaxSplits ? 1 : 2;  // 2: few rows, bf16
     static constexpr KernelId merge[3][3] = {
@@ -1197,7 +1223,7 @@ hipError_t launch_fwd_split(const Params &p, int dtype_bf16, int d, int splits, 
     Params q = p;
     void *args[] = {&q};
     hipError_t e = few ? launch_fwd_few(p, d, splits, stream)
-                       : launch_kernel(kf, dim3(p.B * p.Hq, (p.N + 63) / 64, splits), dim3(256), args, stream);
+                       : launch_kernel(kf, dim3(p.B * p.Hq, (p.N + 16 * nw - 1) / (16 * nw), splits), dim3(64 * nw), args, stream);
     if (e != hipSuccess) return e;
     const size_t rows = (size_t)p.B * p.Hq * p.N;
     int s = splits;

@@ -19,6 +19,7 @@
     X(mxfa_fwd_f64_c) X(mxfa_fwd_f64_n) X(mxfa_fwd_f64_c_g8) X(mxfa_fwd_f64_n_g8)              \
     X(mxfa_fwd_b64_c_w2_q2_pg) X(mxfa_fwd_b64_c_w3_q1_pg) X(mxfa_fwd_b128_c_w2_q1_pg)          \
     X(mxfa_fwd_f64_c_pg) X(mxfa_fwd_f64_c_pg_g8)                                              \
+    X(mxfa_fwd_f64_c_sp_g8) X(mxfa_fwd_f64_c_pg_sp_g8)                                        \
     X(mxfa_fwd_b64_c_w3_q1_sp) X(mxfa_fwd_b128_c_w2_q1_sp) X(mxfa_fwd_f64_c_sp)                \
     X(mxfa_fwd_b64_c_w3_q1_pg_sp) X(mxfa_fwd_b128_c_w2_q1_pg_sp) X(mxfa_fwd_f64_c_pg_sp)       \
     X(mxfa_fwd_merge8_b64) X(mxfa_fwd_merge8_b128) X(mxfa_fwd_merge8_f64)                     \

@@ -48,10 +48,11 @@ hipError_t launch_fwd(const Params &p, int dtype_bf16, int d, int causal, hipStr
 // merging launch: the split count for a shape (1: no split pays), the fp32
 // partials it needs in p.fwd_part, and the two launches (2 <= splits <= 32,
 // or 128 of a few-row shape; K/V contiguous, or through p.block_table).
-// fwd_splits_in: of `splits`, those a workspace of `bytes` holds the partials
-// of, where they are all of them or at least 32 (0: too small).
+// fwd_splits_in: of those, the ones a workspace of `bytes` holds the partials
+// of, where it is all of them or as many as 64-query work-groups take (at most
+// 32; 1, unsplit, where those take none); 0: too small.
 int fwd_splits(const Params &p, int dtype_bf16, int d);
-int fwd_splits_in(const Params &p, int d, int splits, size_t bytes);
+int fwd_splits_in(const Params &p, int dtype_bf16, int d, size_t bytes);
 size_t fwd_split_workspace_bytes(const Params &p, int d, int splits);
 hipError_t launch_fwd_split(const Params &p, int dtype_bf16, int d, int splits, hipStream_t stream);
 hipError_t launch_preprocess(const Params &p, int dtype_bf16, int d, hipStream_t stream);

@@ -486,12 +486,12 @@ int paged_params(const mxfa_prefill_shape *s, const void *q, const void *kcache,
 int run_prefill_maybe_split(const mxfa_prefill_shape *s, Params p, void *workspace, size_t workspace_bytes,
                             void *stream) {
     const int dtype_bf16 = s->dtype == MXFA_BF16;
-    int splits = mxfa::fwd_splits(p, dtype_bf16, s->head_dim);
-    if (splits <= 1)  // the unsplit launch: no workspace needed or read
+    const size_t have = workspace != nullptr && aligned16(workspace) ? workspace_bytes : 0;
+    const int splits = mxfa::fwd_splits_in(p, dtype_bf16, s->head_dim, have);
+    if (splits == 1)  // the unsplit launch: no workspace needed or read
         return from_hip(mxfa::launch_fwd(p, dtype_bf16, s->head_dim, 1, static_cast<hipStream_t>(stream)));
     if (workspace == nullptr) return MXFA_ERR_NULL;
     if (!aligned16(workspace)) return MXFA_ERR_ALIGN;
-    splits = mxfa::fwd_splits_in(p, s->head_dim, splits, workspace_bytes);
     if (splits == 0) return MXFA_ERR_WORKSPACE;
     p.fwd_part = static_cast<float *>(workspace);
     return from_hip(mxfa::launch_fwd_split(p, dtype_bf16, s->head_dim, splits, static_cast<hipStream_t>(stream)));

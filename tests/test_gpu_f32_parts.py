@@ -134,3 +134,42 @@ def test_backward_outside_the_parts():
     assert np.abs(dq[..., 1:] - rq[..., 1:]).max() <= 64 * TOL
     assert np.abs(dk[:, keep] - rk).max() <= 64 * TOL and np.abs(dv[:, keep] - rv).max() <= 64 * TOL
     assert (dk[:, 77] == 0).all() and (dv[:, 77] == 0).all()
+
+
+@pytest.mark.parametrize("n,nh,nkv,pos0", [(70, 28, 2, 2100), (129, 9, 9, 4000), (256, 32, 4, 1000)])
+def test_chunk_split_over_128_query_blocks(n, nh, nkv, pos0):
+    """An fp32 chunk whose keys are split over 8-wave work-groups: contiguous and
+    paged alike, with the whole workspace, a smaller one and (where 64-query
+    blocks need none, the last shape) none."""
+    import torch
+    import mx230_amd as mx
+    rows = -(-(pos0 + n) // 16) * 16
+    rng = np.random.default_rng(n)
+    q, k, v = (rng.standard_normal((r, c * 64)).astype(np.float32) for r, c in ((n, nh), (rows, nkv), (rows, nkv)))
+    table = rng.permutation(rows // 16).astype(np.int32)
+    kp, vp = np.empty_like(k), np.empty_like(v)
+    for i, b in enumerate(table):
+        kp[16 * b:16 * b + 16], vp[16 * b:16 * b + 16] = k[16 * i:16 * i + 16], v[16 * i:16 * i + 16]
+    want = np.empty((n, nh * 64))
+    for h in range(nh):
+        c = slice(h // (nh // nkv) * 64, (h // (nh // nkv) + 1) * 64)
+        s = q[:, h * 64:(h + 1) * 64].astype(np.float64) @ k[:pos0 + n, c].T / 8
+        s[np.arange(pos0 + n)[None] > pos0 + np.arange(n)[:, None]] = -np.inf
+        p = np.exp(s - s.max(1, keepdims=True))
+        want[:, h * 64:(h + 1) * 64] = (p / p.sum(1, keepdims=True)) @ v[:pos0 + n, c]
+    tq, tk, tv, tkp, tvp, tt = (torch.from_numpy(x).cuda() for x in (q, k, v, kp, vp, table))
+    need = mx.prefill_workspace_bytes(n, pos0, nh, nkv, 64, False)
+    one = n * nh * 66 * 4
+    assert need >= 2 * one
+    sizes = [need, need - one + 4] + ([16] if n == 256 else [])
+    for size in sizes:
+        ws = torch.empty(size, dtype=torch.uint8, device="cuda")
+        a, b = (torch.empty(n, nh * 64, device="cuda") for _ in range(2))
+        try:
+            mx.run_prefill_split(tq, tk, tv, a, pos0, nh, nkv, workspace=ws)
+        except mx.MxfaError:  # fewer ranges than 64-query blocks take
+            assert size < need
+            continue
+        mx.run_prefill_paged(tq, tkp, tvp, b, tt, 16, pos0, nh, nkv, split=True, workspace=ws)
+        assert torch.equal(a, b)
+        assert _close(a.cpu().numpy(), want)
