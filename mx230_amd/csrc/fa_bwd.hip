@@ -1135,8 +1135,10 @@ __device__ __forceinline__ void bwd_fused_entry(const Params &p) {
 // 6.3e-7, 6.2e-7. The dQ pass at two work-groups per CU with both score tiles'
 // operands read at once: 76 / 798; the dK/dV pass at three spills 78 registers
 // (274 at B4 H12 N1024).
-struct SplitPair {
+struct BwdSplitSmem {
     SplitTile a, b;
+    __attribute__((aligned(16))) float sL[64], sD[2][64];
+    uint32_t flags[4];
 };
 
 // The work-group's rows again in plain fp32 arithmetic, for operands outside
@@ -1171,7 +1173,7 @@ __device__ __forceinline__ void dq_plain(const Params &p, int bh, int qb) {
 
 // dK (unscaled, sign flipped, times kmul) and dV of the work-group's 64 keys
 // over stages [g0, g0 + nsteps) of the group's query heads (dkv_split_entry).
-template <bool CAUSAL>
+template <bool CAUSAL, bool OWN>
 __device__ __forceinline__ void dkv_plain(const Params &p, int bkv, int kb, int g0, int nsteps, float *dK, float *dV,
                                        float kmul) {
     constexpr int D = 64;
@@ -1192,7 +1194,17 @@ __device__ __forceinline__ void dkv_plain(const Params &p, int bkv, int kb, int 
             const size_t r = bh * N + i;
             const float *Q = static_cast<const float *>(p.q) + r * D + c;
             const float *G = static_cast<const float *>(p.dout) + r * D + c;
-            const float pv = fast_exp2(dot16(k, Q) - p.lse[r] * kLog2e), ds = pv * (p.delta[r] - dot16(v, G));
+            float delta;
+            if constexpr (OWN) {
+                delta = 0.f;
+#pragma unroll
+                for (int e = 0; e < 16; ++e)
+                    delta = __builtin_fmaf(G[e], static_cast<const float *>(p.o_in)[r * D + c + e], delta);
+                delta = quad_sum(delta);
+            } else {
+                delta = p.delta[r];
+            }
+            const float pv = fast_exp2(dot16(k, Q) - p.lse[r] * kLog2e), ds = pv * (delta - dot16(v, G));
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 av[e] = __builtin_fmaf(pv, G[e], av[e]);
@@ -1208,22 +1220,15 @@ __device__ __forceinline__ void dkv_plain(const Params &p, int bkv, int kb, int 
     }
 }
 
-// The fp32 dQ pass, grid (B Hq, 64-query blocks).
+// The fp32 dQ work of query block qb (64 rows) of (batch, query head) bh.
 template <bool CAUSAL, bool DELTA>
-__device__ __forceinline__ void dq_split_entry(const Params &p) {
+__device__ __forceinline__ void dq_split_body(const Params &p, int bh, int qb, BwdSplitSmem &sm) {
     constexpr int D = 64, XT = 4, BQ = 64, BK = 64;
     using PL = PolBF16<64>;  // the parts' layout
     using Stage = SplitStage<256>;
-    __shared__ SplitPair sm;
-    __shared__ uint32_t flags[4];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 4, l16 = lane & 15, N = p.N;
-    const int nqb = (N + BQ - 1) / BQ;
-    const int i = (int)(blockIdx.y * gridDim.x + blockIdx.x);
-    const int rank = CAUSAL ? cu_order_wg(i, p.cu_run, p.cu_runs) : i;  // heaviest first, balanced per CU
-    const int qb = CAUSAL ? nqb - 1 - rank / (int)gridDim.x : rank / (int)gridDim.x;
-    const int bh = rank % (int)gridDim.x;
     const int b = bh / p.Hq, kvh = bh % p.Hq / p.group;
     const size_t kvoff = ((size_t)b * p.Hkv + kvh) * N * D;
     const float *K = static_cast<const float *>(p.k) + kvoff, *V = static_cast<const float *>(p.v) + kvoff;
@@ -1329,7 +1334,7 @@ __device__ __forceinline__ void dq_split_entry(const Params &p) {
     float z = 0.f;
 #pragma unroll
     for (int xt = 0; xt < XT; ++xt) z += zero_of(acc[xt]);
-    if (any_nonfinite<4>(z, flags, wave, lane)) {
+    if (any_nonfinite<4>(z, sm.flags, wave, lane)) {
         dq_plain<CAUSAL>(p, bh, qb);
     } else if (qi < N) {
         float *row = static_cast<float *>(p.dq) + qrow * D;
@@ -1339,17 +1344,23 @@ __device__ __forceinline__ void dq_split_entry(const Params &p) {
     wg_time_after_stores();
 }
 
-// The fp32 dK/dV pass, a 1-D grid of dkv_work's work-groups (64 keys each).
-template <bool CAUSAL>
-__device__ __forceinline__ void dkv_split_entry(const Params &p) {
+// The fp32 dQ pass, grid (B Hq, 64-query blocks).
+template <bool CAUSAL, bool DELTA>
+__device__ __forceinline__ void dq_split_entry(const Params &p) {
+    __shared__ BwdSplitSmem sm;
+    const int nqb = (p.N + 63) / 64, i = (int)(blockIdx.y * gridDim.x + blockIdx.x);
+    const int rank = CAUSAL ? cu_order_wg(i, p.cu_run, p.cu_runs) : i;  // heaviest first, balanced per CU
+    const int qb = CAUSAL ? nqb - 1 - rank / (int)gridDim.x : rank / (int)gridDim.x;
+    dq_split_body<CAUSAL, DELTA>(p, rank % (int)gridDim.x, qb, sm);
+}
+
+// The fp32 dK/dV work wk (dkv_work, 64 keys). OWN: Delta = rowsum(dO O) of each
+// stage's rows is computed here from O, not read from p.delta.
+template <bool CAUSAL, bool OWN>
+__device__ __forceinline__ void dkv_split_body(const Params &p, const DkvWork wk, BwdSplitSmem &sm) {
     constexpr int D = 64, XT = 4, BKV = 64, BQ = 64;
     using PL = PolBF16<64>;
     using Stage = SplitStage<256>;
-    __shared__ SplitPair sm;
-    __shared__ __attribute__((aligned(16))) float sL[BQ], sD[BQ];
-    __shared__ uint32_t flags[4];
-    const DkvWork wk = dkv_work(p, blockIdx.x, BKV, BQ, CAUSAL);
-    if (wk.kb * BKV >= p.N) return;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 4, l16 = lane & 15, N = p.N;
@@ -1377,17 +1388,18 @@ __device__ __forceinline__ void dkv_split_entry(const Params &p) {
     int ld_i = g0 % nqs;
     Stage xq, xg;
     float xl = 0.f;  // waves 0 and 1: LSE and Delta of row `lane`
+    size_t off[Stage::NK];
     auto load = [&]() __attribute__((always_inline)) {
         const int qs = qstart + ld_i * BQ;
 #pragma unroll
         for (int k = 0; k < Stage::NK; ++k) {
-            const size_t off = (ld_row + min(qs + srow[k], N - 1)) * D + scol[k];
-            xq.load(k, static_cast<const float *>(p.q) + off);
-            xg.load(k, static_cast<const float *>(p.dout) + off);
+            off[k] = (ld_row + min(qs + srow[k], N - 1)) * D + scol[k];
+            xq.load(k, static_cast<const float *>(p.q) + off[k]);
+            xg.load(k, static_cast<const float *>(p.dout) + off[k]);
         }
         // rows past N: LSE = +inf makes their p (and so dS) exactly 0
         if (wave == 0) xl = qs + lane < N ? p.lse[ld_row + qs + lane] : INFINITY;
-        if (wave == 1) xl = p.delta[ld_row + min(qs + lane, N - 1)];
+        if (!OWN && wave == 1) xl = p.delta[ld_row + min(qs + lane, N - 1)];
         if (++ld_i == nqs) {
             ld_i = 0;
             ld_row += N;
@@ -1431,8 +1443,9 @@ __device__ __forceinline__ void dkv_split_entry(const Params &p) {
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
                 const int q4 = 32 * blk + PL::bidx(t, g, 0);
-                const f32x4 nl = *reinterpret_cast<const f32x4 *>(sL + q4);
-                const f32x4 dl = *reinterpret_cast<const f32x4 *>(sD + q4);
+                const f32x4 nl = *reinterpret_cast<const f32x4 *>(sm.sL + q4);
+                f32x4 dl = *reinterpret_cast<const f32x4 *>(sm.sD[0] + q4);
+                if constexpr (OWN) dl += *reinterpret_cast<const f32x4 *>(sm.sD[1] + q4);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const float pv = fast_exp2(s[t][0][r] + nl[r]);
@@ -1453,10 +1466,35 @@ __device__ __forceinline__ void dkv_split_entry(const Params &p) {
     int pos = g0 % nqs;  // the stage's place in its query head; the head's first is its diagonal
     for (int st = 0; st < nsteps; ++st) {
         if (st > 0) barrier_lds();
+        f32x4 o[OWN ? Stage::NK : 1][2];
+        if constexpr (OWN) {
+#pragma unroll
+            for (int k = 0; k < Stage::NK; ++k) {
+                const float *src = static_cast<const float *>(p.o_in) + off[k];
+                o[k][0] = *reinterpret_cast<const f32x4 *>(src);
+                o[k][1] = *reinterpret_cast<const f32x4 *>(src + 4);
+            }
+        }
         xq.write(sm.a, tid);
         xg.write(sm.b, tid);
-        if (wave == 0) sL[lane] = -xl * kLog2e;
-        if (wave == 1) sD[lane] = xl;
+        if (wave == 0) sm.sL[lane] = -xl * kLog2e;
+        if constexpr (OWN) {
+            // a row's chunks: two of each lane pair, the pair's and those of the
+            // pair 128 threads on
+            float d = 0.f;
+#pragma unroll
+            for (int k = 0; k < Stage::NK; ++k) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    d = __builtin_fmaf(xg.x[k][0][e], o[k][0][e], d);
+                    d = __builtin_fmaf(xg.x[k][1][e], o[k][1][e], d);
+                }
+            }
+            d += __shfl_xor(d, 1, 64);
+            if ((tid & 1) == 0) sm.sD[tid >> 7][srow[0]] = d;
+        } else {
+            if (wave == 1) sm.sD[0][lane] = xl;
+        }
         if (st + 1 < nsteps) load();
         barrier_lds();
         if (st == 0) wg_time(1);
@@ -1474,8 +1512,8 @@ __device__ __forceinline__ void dkv_split_entry(const Params &p) {
     float z = 0.f;
 #pragma unroll
     for (int xt = 0; xt < XT; ++xt) z += zero_of(accK[xt]) + zero_of(accV[xt]);
-    if (any_nonfinite<4>(z, flags, wave, lane)) {
-        dkv_plain<CAUSAL>(p, wk.bkv, wk.kb, g0, nsteps, dK, dV, kmul);
+    if (any_nonfinite<4>(z, sm.flags, wave, lane)) {
+        dkv_plain<CAUSAL, OWN>(p, wk.bkv, wk.kb, g0, nsteps, dK, dV, kmul);
     } else if (key < N) {
 #pragma unroll
         for (int xt = 0; xt < XT; ++xt) {
@@ -1484,6 +1522,32 @@ __device__ __forceinline__ void dkv_split_entry(const Params &p) {
         }
     }
     wg_time_after_stores();
+}
+
+// The fp32 dK/dV pass, a 1-D grid of dkv_work's work-groups (64 keys each).
+template <bool CAUSAL>
+__device__ __forceinline__ void dkv_split_entry(const Params &p) {
+    __shared__ BwdSplitSmem sm;
+    const DkvWork wk = dkv_work(p, blockIdx.x, 64, 64, CAUSAL);
+    if (wk.kb * 64 >= p.N) return;
+    dkv_split_body<CAUSAL, false>(p, wk, sm);
+}
+
+// Both fp32 passes in one launch: work-groups [0, fused_ndq) the dQ work
+// (which writes Delta), the rest the dK/dV work, which computes its own Delta
+// and so waits for nothing.
+template <bool CAUSAL>
+__device__ __forceinline__ void bwd_split_entry(const Params &p) {
+    __shared__ BwdSplitSmem sm;
+    const int bid = blockIdx.x, nbh = p.B * p.Hq;
+    if (bid < p.fused_ndq) {
+        const int nqb = (p.N + 63) / 64;
+        dq_split_body<CAUSAL, true>(p, bid % nbh, CAUSAL ? nqb - 1 - bid / nbh : bid / nbh, sm);
+    } else {
+        const DkvWork wk = dkv_work(p, bid - p.fused_ndq, 64, 64, CAUSAL);
+        if (wk.kb * 64 >= p.N) return;
+        dkv_split_body<CAUSAL, true>(p, wk, sm);
+    }
 }
 
 // dK / dV of a split dK/dV pass: for each key row, the sum of its key block's
@@ -1551,6 +1615,8 @@ using DkvB128 = DkvTile16<PolBF16<128>, 1>;
     extern "C" __global__ __launch_bounds__(256, DqF32::kWaves) void NAME(Params p) { dq_split_entry<CAUSAL, DELTA>(p); }
 #define MXFA_DKV_F(NAME, CAUSAL)                                                                         \
     extern "C" __global__ __launch_bounds__(256, DkvF32::kWaves) void NAME(Params p) { dkv_split_entry<CAUSAL>(p); }
+#define MXFA_BWD_F(NAME, CAUSAL)                                                                         \
+    extern "C" __global__ __launch_bounds__(256, DkvF32::kWaves) void NAME(Params p) { bwd_split_entry<CAUSAL>(p); }
 #define MXFA_FUSED(NAME, DQT, DKVT, CAUSAL)                                                              \
     extern "C" __global__ __launch_bounds__(256, DKVT::kWaves < DQT::kWaves ? DKVT::kWaves : DQT::kWaves) void \
     NAME(Params p) {                                                                                     \
@@ -1584,6 +1650,8 @@ MXFA_DKV(mxfa_dkv_b128_c, DkvB128, true)
 MXFA_DKV(mxfa_dkv_b128_n, DkvB128, false)
 MXFA_DKV_F(mxfa_dkv_f64_c, true)
 MXFA_DKV_F(mxfa_dkv_f64_n, false)
+MXFA_BWD_F(mxfa_bwd_f64_c, true)
+MXFA_BWD_F(mxfa_bwd_f64_n, false)
 MXFA_FUSED(mxfa_bwd_b64_c, DqB64, DkvB64, true)
 MXFA_FUSED(mxfa_bwd_b64_n, DqB64, DkvB64, false)
 MXFA_FUSED(mxfa_bwd_b64_c_p2, DqB64, DkvB64P2, true)
@@ -1601,6 +1669,7 @@ MXFA_REDUCE(mxfa_dkv_reduce_f32, float)
 #undef MXFA_DKV
 #undef MXFA_DQ_F
 #undef MXFA_DKV_F
+#undef MXFA_BWD_F
 #undef MXFA_FUSED
 #undef MXFA_REDUCE
 #endif
@@ -1955,6 +2024,27 @@ static hipError_t launch_dkv_k(Params p, int causal, hipStream_t stream) {
     const hipError_t e = launch_kernel(id, dim3((unsigned)n), dim3(256), args, stream);
     if (e != hipSuccess || p.dkv_split == 1) return e;
     return launch_dkv_reduce<K>(p, causal, stream);
+}
+
+bool bwd_f32_together(const Params &p, int dtype_bf16, int d, int causal) {
+    if (dtype_bf16 || d != 64 || g_one_launch.load() == 0) return false;
+    Params q = p;
+    dkv_plan_t<DkvF32>(q, causal != 0);
+    if (q.dkv_ws == nullptr) q.dkv_split = 1;
+    return (long long)p.B * p.Hq * ((p.N + 63) / 64) + dkv_work_groups(q, causal != 0, 64) <= 512;
+}
+
+hipError_t launch_bwd_f32(Params p, int causal, hipStream_t stream) {
+    dkv_plan_t<DkvF32>(p, causal != 0);
+    if (p.dkv_ws == nullptr) p.dkv_split = 1;
+    if (p.dkv_split == 1) p.dkv_ws = nullptr;
+    p.fused_ndq = p.B * p.Hq * ((p.N + 63) / 64);
+    p.fused_ndkv = (int)dkv_work_groups(p, causal != 0, 64);
+    void *args[] = {&p};
+    const hipError_t e = launch_kernel(causal ? k_mxfa_bwd_f64_c : k_mxfa_bwd_f64_n,
+                                       dim3((unsigned)(p.fused_ndq + p.fused_ndkv)), dim3(256), args, stream);
+    if (e != hipSuccess || p.dkv_split == 1) return e;
+    return launch_dkv_reduce<KernelsF64>(p, causal, stream);
 }
 
 hipError_t launch_bwd_dkv(const Params &p, int dtype_bf16, int d, int causal, hipStream_t stream) {

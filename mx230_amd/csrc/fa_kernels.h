@@ -33,6 +33,7 @@
     X(mxfa_dq_b128_c) X(mxfa_dq_b128_c_d) X(mxfa_dq_b128_n) X(mxfa_dq_b128_n_d)               \
     X(mxfa_dq_f64_c) X(mxfa_dq_f64_c_d) X(mxfa_dq_f64_n) X(mxfa_dq_f64_n_d)                   \
     X(mxfa_dkv_b64_c) X(mxfa_dkv_b64_n) X(mxfa_dkv_b128_c) X(mxfa_dkv_b128_n)                 \
+    X(mxfa_bwd_f64_c) X(mxfa_bwd_f64_n)                                                       \
     X(mxfa_dkv_f64_c) X(mxfa_dkv_f64_n) X(mxfa_dkv_b64_c_p2) X(mxfa_dkv_b64_n_p2)             \
     X(mxfa_bwd_b64_c) X(mxfa_bwd_b64_n) X(mxfa_bwd_b128_c) X(mxfa_bwd_b128_n)                 \
     X(mxfa_bwd_b64_c_p2) X(mxfa_bwd_b64_n_p2)                                                 \

@@ -74,6 +74,12 @@ size_t dkv_workspace_bytes(const Params &p, int dtype_bf16, int d, int causal);
 // for the shape, and launched with its own epoch.
 bool bwd_fused_available(const Params &p, int dtype_bf16, int d, hipStream_t stream);
 hipError_t launch_bwd_fused(const Params &p, int d, int causal, hipStream_t stream);
+// The fp32 backward from O with both passes in one launch (no flags and no
+// waits: the dK/dV work computes its own Delta), for grids that fit the GPU at
+// once, where the passes then run side by side; with p.dkv_ws a GQA split and
+// its reduce launch, as launch_bwd_dkv.
+bool bwd_f32_together(const Params &p, int dtype_bf16, int d, int causal);
+hipError_t launch_bwd_f32(Params p, int causal, hipStream_t stream);
 // Process-wide settings of the one-launch backward: whether it is used where
 // available, and the bound of each Delta wait in microseconds (< 0: never
 // wait, always compute Delta); read at every launch.

@@ -274,12 +274,14 @@ int mxfa_run_bwd_ws(const mxfa_shape *shape, const void *q, const void *k, const
     {
         // the dQ and dK/dV work in one launch (plus the reduce of a GQA split)
         Params p = bwd_params(shape, q, k, v, dout, lse, delta);
+        p.o_in = o;
+        p.dq = dq;
+        p.dk = dk;
+        p.dv = dv;
+        p.dkv_ws = static_cast<float *>(workspace);
+        if (mxfa::bwd_f32_together(p, shape->dtype == MXFA_BF16, shape->d, shape->causal))
+            return from_hip(mxfa::launch_bwd_f32(p, shape->causal, static_cast<hipStream_t>(stream)));
         if (mxfa::bwd_fused_available(p, shape->dtype == MXFA_BF16, shape->d, static_cast<hipStream_t>(stream))) {
-            p.o_in = o;
-            p.dq = dq;
-            p.dk = dk;
-            p.dv = dv;
-            p.dkv_ws = static_cast<float *>(workspace);
             return from_hip(mxfa::launch_bwd_fused(p, shape->d, shape->causal, static_cast<hipStream_t>(stream)));
         }
     }
