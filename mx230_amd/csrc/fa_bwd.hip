@@ -2026,12 +2026,17 @@ static hipError_t launch_dkv_k(Params p, int causal, hipStream_t stream) {
     return launch_dkv_reduce<K>(p, causal, stream);
 }
 
+// Up to 1.5 times the 512 work-groups that fit at once: us, together against one
+// after the other, 4 work-groups each (non-causal B1 H1 N256) 20 / 36, 64 each
+// (B1 H4 N1024 causal) 69 / 110, 256 each (B1 H8 N2048) 173 / 210, 384 each
+// (B1 H12 N2048) 175 / 227; at 768 each (B4 H12 N1024) 171 / 156: the dQ work runs at the
+// dK/dV work's two work-groups per CU here, not its own three.
 bool bwd_f32_together(const Params &p, int dtype_bf16, int d, int causal) {
     if (dtype_bf16 || d != 64 || g_one_launch.load() == 0) return false;
     Params q = p;
     dkv_plan_t<DkvF32>(q, causal != 0);
     if (q.dkv_ws == nullptr) q.dkv_split = 1;
-    return (long long)p.B * p.Hq * ((p.N + 63) / 64) + dkv_work_groups(q, causal != 0, 64) <= 512;
+    return (long long)p.B * p.Hq * ((p.N + 63) / 64) + dkv_work_groups(q, causal != 0, 64) <= 768;
 }
 
 hipError_t launch_bwd_f32(Params p, int causal, hipStream_t stream) {

@@ -777,52 +777,55 @@ __device__ __forceinline__ void stage_kv(typename Pol::T *sk, typename Pol::T *s
     stage_rows<Pol, NT>(sv, V + (size_t)k0 * row_stride, N - k0, pl, wave, row_stride);
 }
 
-// A paged K/V stage (Params::block_table): per staging load of the thread,
-// the block-table entry of its row in the next stage to be staged. fetch()
-// loads them for the stage at k0 (rows past N take row N - 1, as stage_rows
-// does); stage() issues that stage's loads from them. A caller fetches one
-// stage ahead of the loads, so the table loads complete within the stage
-// before and the staging loads never wait for them.
+// A paged K/V stage (Params::block_table): the block-table entries of the
+// thread's rows in the next stage to be staged. fetch() loads them for the stage
+// at k0 (rows past N take row N - 1, as stage_rows does); stage() issues that
+// stage's loads from them. A caller fetches one stage ahead of the loads, so the
+// table loads complete within the stage before and the staging loads never wait
+// for them. Load k NT + tid of a tile is at slot (k NT + tid) % 128 / 2 of its
+// column group, so a thread's loads are of NR rows in turn (one row for 128
+// threads and more): one table entry and one row address serve them all, where
+// an entry and an address per load cost the 128-query kernel its third wave per
+// SIMD (4096 tokens of 32/4 heads 87.8 -> 81.9 us a call, 8000 of 14/2 141 ->
+// 129, 2000 of 32/8 d = 128 54 -> 48).
 template <class Pol, int NT = 256>
 struct PagedRows {
-    static constexpr int NK = RowPlan<Pol, NT>::NK;
-    int blk[NK];
+    static constexpr int NK = RowPlan<Pol, NT>::NK, NR = NT >= 128 ? 1 : 128 / NT;
+    static_assert(Pol::ROWS == 64 && NK % NR == 0, "128 chunks to a column group");
+    int blk[NR];
 
     __device__ __forceinline__ void fetch(const int *bt, int shift, int k0, int N, const RowPlan<Pol, NT> &pl) {
 #pragma unroll
-        for (int k = 0; k < NK; ++k) {
-            const int t = min(k0 + (int)(pl.rc[k] & 255u), N - 1);
-            blk[k] = bt[t >> shift];
-        }
+        for (int r = 0; r < NR; ++r) blk[r] = bt[min(k0 + (int)(pl.rc[r] & 255u), N - 1) >> shift];
     }
-    // rows k0 .. k0 + Pol::ROWS - 1 of K and V (cache rows row_stride
-    // elements apart) into the LDS tiles, as stage_kv does for a contiguous cache
-    __device__ __forceinline__ void stage(typename Pol::T *sk, typename Pol::T *sv, const typename Pol::T *K,
-                                          const typename Pol::T *V, int k0, int N, int shift,
-                                          const RowPlan<Pol, NT> &pl, int wave, int row_stride) const {
-        const uint32_t bk = lds_addr(sk) + wave * 64 * 16, bv = lds_addr(sv) + wave * 64 * 16;
-        const int mask = (1 << shift) - 1;
-#pragma unroll
-        for (int k = 0; k < NK; ++k) {
-            const int t = min(k0 + (int)(pl.rc[k] & 255u), N - 1);
-            const size_t off = (((size_t)blk[k] << shift) + (size_t)(t & mask)) * (size_t)row_stride +
-                               (pl.rc[k] >> 8) / sizeof(typename Pol::T);
-            lds_dma16(bk + k * NT * 16, K + off);
-            lds_dma16(bv + k * NT * 16, V + off);
-        }
+    // the first element of row r's cache row, from the tensor's base
+    __device__ __forceinline__ size_t row(int r, int k0, int N, int shift, const RowPlan<Pol, NT> &pl,
+                                          int row_stride) const {
+        const int t = min(k0 + (int)(pl.rc[r] & 255u), N - 1);
+        return (((size_t)blk[r] << shift) + (size_t)(t & ((1 << shift) - 1))) * (size_t)row_stride;
     }
-    // the same rows of one tensor
+    // rows k0 .. k0 + Pol::ROWS - 1 of X (cache rows row_stride elements apart)
+    // into an LDS tile, as stage_rows does for a contiguous cache
     __device__ __forceinline__ void stage_one(typename Pol::T *tile, const typename Pol::T *X, int k0, int N, int shift,
                                               const RowPlan<Pol, NT> &pl, int wave, int row_stride) const {
         const uint32_t base = lds_addr(tile) + wave * 64 * 16;
-        const int mask = (1 << shift) - 1;
+        const typename Pol::T *src[NR];
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+            src[r] = X + row(r, k0, N, shift, pl, row_stride) + (pl.rc[r] >> 8) / sizeof(typename Pol::T);
 #pragma unroll
         for (int j = 0; j < NK; ++j) {
+            // NR loads on, the row's chunk is NR NT / 128 column groups of 16 on
             const int k = load_order<NT, NK>(j);
-            const int t = min(k0 + (int)(pl.rc[k] & 255u), N - 1);
-            lds_dma16(base + k * NT * 16, X + ((((size_t)blk[k] << shift) + (size_t)(t & mask)) * (size_t)row_stride +
-                                               (pl.rc[k] >> 8) / sizeof(typename Pol::T)));
+            lds_dma16(base + k * NT * 16, src[k % NR] + (k - k % NR) * NT / 8);
         }
+    }
+    // the same rows of K and V
+    __device__ __forceinline__ void stage(typename Pol::T *sk, typename Pol::T *sv, const typename Pol::T *K,
+                                          const typename Pol::T *V, int k0, int N, int shift,
+                                          const RowPlan<Pol, NT> &pl, int wave, int row_stride) const {
+        stage_one(sk, K, k0, N, shift, pl, wave, row_stride);
+        stage_one(sv, V, k0, N, shift, pl, wave, row_stride);
     }
 };
 

@@ -1004,10 +1004,10 @@ MXFA_FWD_F(mxfa_fwd_f64_c_pg_sp, 4, true, true, true)
 MXFA_FWD_F(mxfa_fwd_f64_c_sp_g8, 8, true, false, true)
 MXFA_FWD_F(mxfa_fwd_f64_c_pg_sp_g8, 8, true, true, true)
 // the prefill over a paged cache (causal, as the prefill always is)
-// (the table entries take registers: the three-wave 128-query d = 64 and the
-// 128-query d = 128 forms would spill in their loops, so paged launches use
-// two waves at d = 64 and 64-query work-groups at d = 128)
+// (the table entry and row address take registers: the 128-query d = 128 form
+// would spill, so paged launches use 64-query work-groups there)
 MXFA_FWD_PG(mxfa_fwd_b64_c_w2_q2_pg, PolBF16<64>, 2, 2)
+MXFA_FWD_PG(mxfa_fwd_b64_c_w3_q2_pg, PolBF16<64>, 3, 2)
 MXFA_FWD_PG(mxfa_fwd_b64_c_w3_q1_pg, PolBF16<64>, 3, 1)
 MXFA_FWD_PG(mxfa_fwd_b128_c_w2_q1_pg, PolBF16<128>, 2, 1)
 // the prefill split over its keys (causal, 64-query work-groups) and the
@@ -1062,7 +1062,8 @@ MXFA_FWD_FEW(mxfa_fwd_b128_few_pg_sp, 128, 4, true, true)
 template <class Pol, bool CAUSAL>
 static KernelId fwd_kernel_id(int wps, int qt, bool paged) {
     if constexpr (Pol::D == 64) {
-        if (CAUSAL && paged) return qt == 1 ? k_mxfa_fwd_b64_c_w3_q1_pg : k_mxfa_fwd_b64_c_w2_q2_pg;
+        if (CAUSAL && paged)
+            return qt == 1 ? k_mxfa_fwd_b64_c_w3_q1_pg : wps == 3 ? k_mxfa_fwd_b64_c_w3_q2_pg : k_mxfa_fwd_b64_c_w2_q2_pg;
         if (CAUSAL) return qt == 1 ? k_mxfa_fwd_b64_c_w3_q1 : wps == 3 ? k_mxfa_fwd_b64_c_w3_q2 : k_mxfa_fwd_b64_c_w2_q2;
         return qt == 1 ? k_mxfa_fwd_b64_n_w3_q1 : k_mxfa_fwd_b64_n_w2_q2;
     } else {
@@ -1078,8 +1079,8 @@ static hipError_t launch_fwd_qt(Params p, hipStream_t stream) {
     constexpr int kHi = Pol::kWavesFwdCausal;
     int wps = QT == 1 ? kHi : Pol::kWaves;
     if constexpr (CAUSAL && kHi > Pol::kWaves && QT > 1) {
-        // enough causal work-groups to fill kHi per CU (256 CUs); not paged
-        if ((long long)grid.x * grid.y >= 256LL * kHi && p.block_table == nullptr) wps = kHi;
+        // enough causal work-groups to fill kHi per CU (256 CUs)
+        if ((long long)grid.x * grid.y >= 256LL * kHi) wps = kHi;
     }
     const KernelId id = fwd_kernel_id<Pol, CAUSAL>(wps, QT, p.block_table != nullptr);
     if (CAUSAL) cu_balance(&p, id, (long long)grid.x * grid.y);
