@@ -158,9 +158,9 @@ int mxfa_run_bwd_flash(const mxfa_shape *shape, const void *q, const void *k, co
 int mxfa_run_bwd_dq_delta(const mxfa_shape *shape, const void *q, const void *k, const void *v, const void *o,
                           const void *dout, const float *lse, float *delta, void *dq, void *stream);
 
-/* The whole backward from O in two launches: the dQ pass computes
- * Delta = rowsum(dO * O) itself (writing it to `delta`, B*Hq*N fp32, which the
- * caller owns as for mxfa_run_preprocess) and the dK/dV pass reads it.
+/* The whole backward from O in two launches, or one (below): the dQ pass
+ * computes Delta = rowsum(dO * O) itself (writing it to `delta`, B*Hq*N fp32,
+ * which the caller owns as for mxfa_run_preprocess) and the dK/dV pass reads it.
  * Replaces the sequence run_preprocess + run_bwd_flash (main.rs:126-143,
  * :179-210; attention_bwd.cu:32-44, :96-243) with the preprocess launch folded
  * into the dQ pass; results equal that sequence's up to the summation order of
@@ -181,7 +181,11 @@ int mxfa_run_bwd(const mxfa_shape *shape, const void *q, const void *k, const vo
  * work-groups, so the results equal the two-launch form's bitwise either way.
  * mxfa_bwd_options.one_launch = 0 selects two launches, and so does a stream
  * under graph capture (a replayed launch would reuse the capture's flag
- * epoch); this query answers for an ordinary stream.
+ * epoch); this query answers for an ordinary stream. An fp32 grid that fits the
+ * GPU about at once also takes one launch unless one_launch = 0 (the dK/dV
+ * work-groups compute Delta themselves, with no flags, captured or not; dK
+ * and dV then equal the two launches' to fp32 rounding of Delta); this query
+ * is 0 for it.
  * No counterpart in the reference: it tells callers (and benchmarks) which
  * kernels the backward from O (main.rs:126-143, :179-210) becomes. */
 int mxfa_bwd_one_launch(const mxfa_shape *shape);

@@ -364,7 +364,8 @@ def run_bwd(q, k, v, o, do, lse, delta, dq, dk, dv, causal: bool, scale: float =
     """The whole backward from O (mxfa_run_bwd): the dQ work computes
     Delta = rowsum(dO * O) itself and writes it to ``delta`` for the dK/dV
     work (run_preprocess + run_bwd_flash with the preprocess launch folded in);
-    one launch for bf16 (bwd_one_launch), else two. Outputs are overwritten."""
+    one launch for bf16 (bwd_one_launch) and small fp32 grids, else two.
+    Outputs are overwritten."""
     _invoke(*_call_bwd(q, k, v, o, do, lse, delta, dq, dk, dv, causal, scale, stream))
 
 
