@@ -10,6 +10,7 @@
 
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cstdint>
@@ -97,16 +98,13 @@ bool shape_of(const at::Tensor *q, const at::Tensor *k, const at::Tensor *v, PyO
 
 PyObject *status(int rc) { return PyLong_FromLong(rc); }
 
+// Runs f; a C++ exception becomes the Python one torch gives it (its
+// OutOfMemoryError among them).
 template <class F>
 PyObject *guarded(F f) {
-    try {
-        return f();
-    } catch (const python_error &) {  // the Python error is set
-        return nullptr;
-    } catch (const std::exception &e) {
-        if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, e.what());
-        return nullptr;
-    }
+    HANDLE_TH_ERRORS
+    return f();
+    END_HANDLE_TH_ERRORS
 }
 
 // attention_fwd(q, k, v, causal, scale) -> (o, lse)

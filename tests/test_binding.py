@@ -67,3 +67,47 @@ def test_prefill_same_as_python_path(n, pos0):
         mx.run_prefill(q, k[:pos0], v[:pos0], a, pos0, Hq, Hkv, d)
     with pytest.raises(mx.MxfaError):  # a head size the kernels do not have
         mx.run_prefill(q, k, v, a, pos0, Hq, Hkv, 32)
+
+
+@pytest.mark.gpu
+def test_current_stream_and_capture():
+    """The calls run on torch's current stream: captured into a graph there and
+    replayed on new inputs (with eager work between), each replay gives the
+    eager result."""
+    import torch
+    torch.manual_seed(4)
+    shape = (1, 2, 100, 64)
+    q, k, v = (torch.randn(shape, device="cuda") for _ in range(3))
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        mx.attention_fwd(q, k, v, True)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        o, lse = mx.attention_fwd(q, k, v, True)
+        grads = mx.attention_bwd(q, k, v, o, lse, o, True)
+    for _ in range(3):
+        for x in (q, k, v):
+            x.copy_(torch.randn(shape, device="cuda"))
+        g.replay()
+        torch.cuda.synchronize()
+        eo, el = mx.attention_fwd(q, k, v, True)
+        for a, b in zip((o, lse, *grads), (eo, el, *mx.attention_bwd(q, k, v, eo, el, eo, True))):
+            assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+def test_out_of_memory_keeps_its_type():
+    import torch
+    if not hasattr(torch, "OutOfMemoryError"):
+        pytest.skip("this torch has no OutOfMemoryError")
+    q = torch.zeros(1, 1, 128, 64, device="cuda", dtype=torch.bfloat16)
+    torch.cuda.empty_cache()
+    torch.cuda.set_per_process_memory_fraction(1e-6)
+    try:
+        with pytest.raises(torch.OutOfMemoryError):
+            keep = []
+            for _ in range(4096):
+                keep.append(mx.attention_fwd(q, q, q, False))
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
