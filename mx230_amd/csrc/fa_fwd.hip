@@ -1195,6 +1195,7 @@ int fwd_splits(const Params &p, int dtype_bf16, int d) {
 
 int fwd_splits_in(const Params &p, int dtype_bf16, int d, size_t bytes) {
     const int want = fwd_splits(p, dtype_bf16, d), must = fwd_splits_64(p, dtype_bf16, d, kFwdMaxSplits);
+    if (want <= 1) return 1;  // few rows of more than 128 heads: unsplit, where 64-query work-groups split
     const size_t one = (size_t)p.B * p.Hq * p.N * (size_t)(d + 2) * sizeof(float);
     const int fit = (int)std::min<size_t>(bytes / one, (size_t)want);
     if (must <= 1) return std::max(fit, 1);

@@ -295,6 +295,32 @@ def test_prefill_split_argument_checks(lib):
     assert lib.mxfa_run_prefill_paged_ws(ctypes.byref(sh), ok, ok, ok, ok, ok, 16, ok, need - 4, None) == -8
 
 
+@pytest.mark.parametrize("d,dtype", [(64, mx.MXFA_BF16), (128, mx.MXFA_BF16), (64, mx.MXFA_F32)])
+def test_prefill_takes_the_workspace_it_asks_for(lib, d, dtype):
+    """A workspace of the reported size (none, or any, where that is 0) never
+    counts as missing or too small: without a device such a call gets as far as
+    its launch."""
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("made-up device addresses: on hosts without a device only")
+    ok = ctypes.c_void_p(4096)
+    launched = set()
+    for nh, nkv in [(1, 1), (8, 1), (14, 2), (32, 4), (128, 128), (129, 129), (144, 144), (144, 12), (160, 8),
+                    (192, 64), (256, 256), (300, 300), (2400, 150)]:
+        for n in (1, 2, 8, 16, 17, 64, 65, 200, 1000):
+            for pos0 in (0, 500, 1000, 1200, 1900, 2100, 5000, 70000):
+                sh = _prefill(n_tok=n, n_head=nh, n_kv_head=nkv, head_dim=d, pos0=pos0, dtype=dtype,
+                              q_stride=nh * d, kv_stride=nkv * d, out_stride=nh * d)
+                need = lib.mxfa_prefill_workspace_bytes(ctypes.byref(sh))
+                for ws, size in [(ok, need)] + ([(None, 0), (ok, 16)] if need == 0 else []):
+                    rc = (lib.mxfa_run_prefill_ws(ctypes.byref(sh), ok, ok, ok, ok, ws, size, None),
+                          lib.mxfa_run_prefill_paged_ws(ctypes.byref(sh), ok, ok, ok, ok, ok, 16, ws, size, None))
+                    assert not {mx_status("MXFA_ERR_NULL"), mx_status("MXFA_ERR_WORKSPACE")} & set(rc), (
+                        n, nh, nkv, pos0, need, size, rc)
+                    launched.update(rc)
+    assert launched <= {mx_status("MXFA_ERR_LAUNCH"), mx_status("MXFA_ERR_DEVICE"), mx_status("MXFA_ERR_CODE_OBJECT")}
+
+
 def test_probe_argument_checks(lib):
     """The probes validate before launching (no device needed for these)."""
     import ctypes

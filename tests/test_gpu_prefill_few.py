@@ -18,7 +18,9 @@ pytestmark = pytest.mark.gpu
 # 1 token: the GQA group's heads are the rows; 16: the most rows of the kernel
 @pytest.mark.parametrize("n,nh,nkv,pos0", [
     (1, 1, 1, 0), (1, 7, 1, 62), (1, 7, 1, 63), (1, 16, 1, 64), (1, 8, 2, 511), (1, 8, 2, 512), (1, 4, 4, 1023),
-    (1, 14, 2, 1024), (1, 8, 1, 8200), (1, 3, 1, 40000), (16, 2, 1, 100), (16, 2, 1, 1500), (3, 4, 2, 0), (5, 2, 2, 1021)])
+    (1, 14, 2, 1024), (1, 8, 1, 8200), (1, 3, 1, 40000), (16, 2, 1, 100), (16, 2, 1, 1500), (3, 4, 2, 0), (5, 2, 2, 1021),
+    # more than 128 heads of rows: unsplit with any workspace or none
+    (1, 144, 144, 1200), (8, 144, 12, 1200)])
 def test_few_rows(n, nh, nkv, pos0, hd):
     import torch
     import mx230_amd as mx
