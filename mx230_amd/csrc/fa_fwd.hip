@@ -728,7 +728,8 @@ __device__ __forceinline__ void fwd_split_entry(const Params &p) {
     // work-group's first stage, fwd_stage_lazy's: scores relative to m, and
     // m raised only where a lane's sum of p passes kLazySum. A row that precedes
     // every key of the first stage (a key split) has m = -inf, and then
-    // precedes all later ones too.
+    // precedes all later ones too; with finite operands whose first scores all
+    // overflow to -inf it does not, and the rows are run again (below).
     auto compute = [&](auto first, bool edge, int k0) __attribute__((always_inline)) {
         constexpr bool FIRST = decltype(first)::value;
         const float start = FIRST || m == -INFINITY ? 0.f : -m;
@@ -835,6 +836,9 @@ __device__ __forceinline__ void fwd_split_entry(const Params &p) {
     float z = 0.f * ltot;
 #pragma unroll
     for (int xt = 0; xt < XT; ++xt) z += zero_of(acc[xt]);
+    // a row with keys here whose first stage's scores all overflowed to -inf: m
+    // stayed there, and O and the sum hold the later stages relative to 0
+    if (m == -INFINITY && s_lo < s_hi && (!CAUSAL || s_lo * BK <= pos0 + qi)) z = NAN;
     if (any_nonfinite<NW>(z, sm.flags, wave, lane)) {
         fwd_plain<NW, CAUSAL, PAGED, SPLIT>(p, bh, qb, s_lo * BK, s_hi * BK);
     } else if (qi < N) {

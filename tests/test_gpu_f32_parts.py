@@ -83,6 +83,62 @@ def test_forward_outside_the_parts(H):
     assert _close(lse, rl)
 
 
+@pytest.mark.parametrize("H", [2, 171], ids=["g4", "g8"])
+def test_forward_first_keys_overflow(H):
+    """Finite operands whose scores with the first 64 keys all overflow to -inf:
+    O and LSE are those over the other keys."""
+    rng = np.random.default_rng(12)
+    q, k, v = (rng.standard_normal((H, 300, 64)).astype(np.float32) for _ in range(3))
+    q[..., 0] = 1e20
+    k[..., 0] = 0
+    k[:, :64, 0] = -1e20
+    o, lse = _fwd(q, k, v, False)
+    ro, rl = _ref(q, k[:, 64:], v[:, 64:], False)
+    assert _close(o, ro) and _close(lse, rl)
+
+
+@pytest.mark.parametrize("paged", [False, True])
+@pytest.mark.parametrize("n,nh,nkv,pos0", [(300, 2, 2, 0), (70, 28, 2, 2100), (8, 4, 2, 2000)], ids=["whole", "g8", "g4"])
+def test_first_keys_overflow(n, nh, nkv, pos0, paged):
+    """Finite operands whose scores with the first 64 keys (and with those of a
+    later split's first stage) all overflow to -inf: those keys have no weight,
+    and the rows that see others are the softmax over these."""
+    import torch
+    import mx230_amd as mx
+    rng = np.random.default_rng(11)
+    rows = -(-(pos0 + n) // 16) * 16
+    q, k, v = (rng.standard_normal((r, c, 64)).astype(np.float32) for r, c in ((n, nh), (rows, nkv), (rows, nkv)))
+    q[..., 0] = 1e20
+    k[..., 0] = 0
+    gone = np.arange(rows) % 1024 < 64
+    k[gone, :, 0] = -1e20
+    want = np.full((n, nh, 64), np.nan)
+    for h in range(nh):
+        for i in range(n):
+            at = np.flatnonzero(~gone[:pos0 + i + 1])
+            if len(at):
+                s = k[at, h * nkv // nh].astype(np.float64) @ q[i, h] / 8
+                p = np.exp(s - s.max())
+                want[i, h] = (p / p.sum()) @ v[at, h * nkv // nh]
+    seen = ~np.isnan(want[:, 0, 0])
+    assert seen.sum() >= 8
+    table = rng.permutation(rows // 16).astype(np.int32)
+    kp, vp = np.empty_like(k), np.empty_like(v)
+    for i, b in enumerate(table):
+        kp[16 * b:16 * b + 16], vp[16 * b:16 * b + 16] = k[16 * i:16 * i + 16], v[16 * i:16 * i + 16]
+    tq, tk, tv = (torch.from_numpy(x.reshape(len(x), -1)).cuda() for x in (q, kp if paged else k, vp if paged else v))
+    tt = torch.from_numpy(table).cuda()
+    for split in (False, True):
+        o = torch.empty(n, nh * 64, device="cuda")
+        if paged:
+            mx.run_prefill_paged(tq, tk, tv, o, tt, 16, pos0, nh, nkv, split=split)
+        elif split:
+            mx.run_prefill_split(tq, tk, tv, o, pos0, nh, nkv)
+        else:
+            mx.run_prefill(tq, tk, tv, o, pos0, nh, nkv)
+        assert _close(o.cpu().numpy().reshape(n, nh, 64)[seen], want[seen]), split
+
+
 def _ref_bwd(q, k, v, do, causal):
     """float64 dQ, dK, dV (one head per KV head)."""
     q, k, v, do = (x.astype(np.float64) for x in (q, k, v, do))
