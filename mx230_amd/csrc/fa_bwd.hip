@@ -1256,8 +1256,8 @@ __device__ __forceinline__ void dq_split_body(const Params &p, int bh, int qb, B
 
     const size_t qrow = (size_t)bh * N + min(qi, N - 1);
     Split3 qf[2], gf[2];
-    split_row(qf, static_cast<const float *>(p.q) + qrow * D, g, p.scale_log2, qi < N);
-    split_row(gf, static_cast<const float *>(p.dout) + qrow * D, g, -1.0f, qi < N);
+    const bool low = split_row(qf, static_cast<const float *>(p.q) + qrow * D, g, p.scale_log2 * kPartDown, qi < N);
+    split_row(gf, static_cast<const float *>(p.dout) + qrow * D, g, -kPartUp, qi < N);
     // added to the scores and to -dP (-dO in registers) once the products are
     // summed, smallest first: fewer roundings at the size of LSE
     const float nl = qi < N ? -p.lse[qrow] * kLog2e : 0.f;
@@ -1274,7 +1274,7 @@ __device__ __forceinline__ void dq_split_body(const Params &p, int bh, int qb, B
     } else {
         dl = p.delta[qrow];
     }
-    dl = qi < N ? dl : 0.f;
+    dl = qi < N ? dl * kDsUp : 0.f;
     f32x4 acc[XT];
 #pragma unroll
     for (int xt = 0; xt < XT; ++xt) acc[xt] = zero4();
@@ -1310,7 +1310,7 @@ __device__ __forceinline__ void dq_split_body(const Params &p, int bh, int qb, B
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) s[t][0][r] = fast_exp2(s[t][0][r] + nl) * (dp[t][0][r] + dl);  // -dS / scale
+                for (int r = 0; r < 4; ++r) s[t][0][r] = fast_exp2(s[t][0][r] + nl) * (dp[t][0][r] + dl);  // -dS kDsUp / scale
             }
             const Split3 ds[1] = {split3(s[0][0], s[1][0])};
 #pragma unroll
@@ -1331,7 +1331,7 @@ __device__ __forceinline__ void dq_split_body(const Params &p, int bh, int qb, B
         compute(st + 1 == nsteps, st * BK);
     }
     wg_time(2);
-    float z = 0.f;
+    float z = low ? NAN : 0.f;
 #pragma unroll
     for (int xt = 0; xt < XT; ++xt) z += zero_of(acc[xt]);
     if (any_nonfinite<4>(z, sm.flags, wave, lane)) {
@@ -1339,7 +1339,7 @@ __device__ __forceinline__ void dq_split_body(const Params &p, int bh, int qb, B
     } else if (qi < N) {
         float *row = static_cast<float *>(p.dq) + qrow * D;
 #pragma unroll
-        for (int xt = 0; xt < XT; ++xt) store4<float>(row + 16 * xt + 4 * g, acc[xt], -p.scale);
+        for (int xt = 0; xt < XT; ++xt) store4<float>(row + 16 * xt + 4 * g, acc[xt] * (kDsDown * kPartDown), -p.scale);
     }
     wg_time_after_stores();
 }
@@ -1408,8 +1408,8 @@ __device__ __forceinline__ void dkv_split_body(const Params &p, const DkvWork wk
     if (nsteps > 0) load();
     Split3 kf[2], vf[2];
     const size_t krow = kvoff + (size_t)min(key, N - 1) * D;
-    split_row(kf, static_cast<const float *>(p.k) + krow, g, p.scale_log2, key < N);
-    split_row(vf, static_cast<const float *>(p.v) + krow, g, -1.0f, key < N);
+    const bool low = split_row(kf, static_cast<const float *>(p.k) + krow, g, p.scale_log2 * kPartDown, key < N);
+    split_row(vf, static_cast<const float *>(p.v) + krow, g, -kPartUp, key < N);
     f32x4 accK[XT], accV[XT];
 #pragma unroll
     for (int xt = 0; xt < XT; ++xt) accK[xt] = accV[xt] = zero4();
@@ -1450,7 +1450,7 @@ __device__ __forceinline__ void dkv_split_body(const Params &p, const DkvWork wk
                 for (int r = 0; r < 4; ++r) {
                     const float pv = fast_exp2(s[t][0][r] + nl[r]);
                     s[t][0][r] = pv;
-                    dp[t][0][r] = pv * (dp[t][0][r] + dl[r]);  // -dS / scale
+                    dp[t][0][r] = pv * (dp[t][0][r] + dl[r]);  // -dS kDsUp / scale
                 }
             }
             const Split3 cp[1] = {split3(s[0][0], s[1][0])}, cds[1] = {split3(dp[0][0], dp[1][0])};
@@ -1491,9 +1491,9 @@ __device__ __forceinline__ void dkv_split_body(const Params &p, const DkvWork wk
                 }
             }
             d += __shfl_xor(d, 1, 64);
-            if ((tid & 1) == 0) sm.sD[tid >> 7][srow[0]] = d;
+            if ((tid & 1) == 0) sm.sD[tid >> 7][srow[0]] = d * kDsUp;
         } else {
-            if (wave == 1) sm.sD[0][lane] = xl;
+            if (wave == 1) sm.sD[0][lane] = xl * kDsUp;
         }
         if (st + 1 < nsteps) load();
         barrier_lds();
@@ -1509,7 +1509,7 @@ __device__ __forceinline__ void dkv_split_body(const Params &p, const DkvWork wk
     float *dK = part ? p.dkv_ws + (size_t)wk.sp * plane + kvoff : static_cast<float *>(p.dk) + kvoff;
     float *dV = part ? dK + (size_t)p.dkv_split * plane : static_cast<float *>(p.dv) + kvoff;
     const float kmul = part ? 1.0f : -p.scale;
-    float z = 0.f;
+    float z = low ? NAN : 0.f;
 #pragma unroll
     for (int xt = 0; xt < XT; ++xt) z += zero_of(accK[xt]) + zero_of(accV[xt]);
     if (any_nonfinite<4>(z, sm.flags, wave, lane)) {
@@ -1517,8 +1517,8 @@ __device__ __forceinline__ void dkv_split_body(const Params &p, const DkvWork wk
     } else if (key < N) {
 #pragma unroll
         for (int xt = 0; xt < XT; ++xt) {
-            store4<float>(dK + (size_t)key * D + 16 * xt + 4 * g, accK[xt], kmul);
-            store4<float>(dV + (size_t)key * D + 16 * xt + 4 * g, accV[xt], 1.0f);
+            store4<float>(dK + (size_t)key * D + 16 * xt + 4 * g, accK[xt] * (kDsDown * kPartDown), kmul);
+            store4<float>(dV + (size_t)key * D + 16 * xt + 4 * g, accV[xt], kPartDown);
         }
     }
     wg_time_after_stores();

@@ -401,10 +401,23 @@ struct Split3 {
     bf16x8 h, m, l;
 };
 
-//
-// The later parts of an infinity, or of a value that rounds to one in bf16,
-// are NaN (inf - inf): kernels that use parts check their results and, on any
-// that is not finite, run the work-group again in plain fp32 arithmetic.
+// Range: the last part of x is a normal bf16, and the parts are x to 24 bits,
+// from |x| = 2^-103 up. So the operands that pass through LDS (SplitStage) are
+// multiplied by kPartUp, which puts every normal fp32 value there, and what is
+// computed from them by a power of two that undoes it: the registers' operand
+// of their scores by kPartDown (a row of which only smaller values are left is
+// flagged, split_row), those of dP by kPartUp too, which keeps dS (scaled
+// kDsUp then) in range as well, and the sums at the end. Without it V or dO of
+// size 2^-115 gave dQ and dK errors of 9e-6 and of 2^-120, 2.9e-4, instead of
+// 3e-7. It costs 1.3% (causal B4 H12 N1024 forward and backward 185.6 -> 188.0
+// us, 500 tokens after 3584 split 48.9 -> 49.5). The later parts of an infinity, or of a value that rounds to one in
+// bf16 (after kPartUp: from 2^104 on), are NaN (inf - inf). Kernels that use
+// parts check their results and, on any that is not finite or a flagged row,
+// run the work-group again in plain fp32 arithmetic.
+constexpr float kPartUp = 0x1p24f, kPartDown = 0x1p-24f;
+constexpr float kDsUp = 0x1p48f, kDsDown = 0x1p-48f;
+constexpr float kPartMin = 0x1p-102f;
+
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 // One part of a pair: the nearest bf16s, packed, and what is left of each
@@ -509,7 +522,7 @@ struct SplitStage {
     __device__ __forceinline__ void write(SplitTile &t, int tid) const {
 #pragma unroll
         for (int k = 0; k < NK; ++k) {
-            const Split3 s = split3(x[k][0], x[k][1]);
+            const Split3 s = split3(x[k][0] * kPartUp, x[k][1] * kPartUp);
             const int off = (k * NT + tid) * 8;
             *reinterpret_cast<bf16x8 *>(t.part[0] + off) = s.h;
             *reinterpret_cast<bf16x8 *>(t.part[1] + off) = s.m;
@@ -897,14 +910,22 @@ constexpr int tile_loads() {
 }
 
 // A row's two 8-element operands of a lane (k-steps 0 and 1), times mul, as
-// parts; zeros for rows that are not there.
-__device__ __forceinline__ void split_row(Split3 (&f)[2], const float *row, int g, float mul, bool valid) {
+// parts; zeros for rows that are not there. True for the whole wave if all of
+// some row's values are below kPartMin and not all 0: its parts are not 24 bits.
+__device__ __forceinline__ bool split_row(Split3 (&f)[2], const float *row, int g, float mul, bool valid) {
+    float mx = 0.f;
 #pragma unroll
     for (int kc = 0; kc < 2; ++kc) {
-        const f32x4 a = *reinterpret_cast<const f32x4 *>(row + 32 * kc + 8 * g) * mul;
-        const f32x4 b = *reinterpret_cast<const f32x4 *>(row + 32 * kc + 8 * g + 4) * mul;
-        f[kc] = split3(valid ? a : zero4(), valid ? b : zero4());
+        f32x4 a = *reinterpret_cast<const f32x4 *>(row + 32 * kc + 8 * g) * mul;
+        f32x4 b = *reinterpret_cast<const f32x4 *>(row + 32 * kc + 8 * g + 4) * mul;
+        a = valid ? a : zero4();
+        b = valid ? b : zero4();
+#pragma unroll
+        for (int e = 0; e < 4; ++e) mx = fmaxf(mx, fmaxf(fabsf(a[e]), fabsf(b[e])));
+        f[kc] = split3(a, b);
     }
+    mx = xg_max(mx);
+    return __builtin_amdgcn_ballot_w64(mx > 0.f && mx < kPartMin) != 0;
 }
 
 // True for every wave of the work-group if any of its lanes holds a value that

@@ -717,8 +717,8 @@ __device__ __forceinline__ void fwd_split_entry(const Params &p) {
     }
 
     Split3 qf[1][2];
-    split_row(qf[0], static_cast<const float *>(p.q) + b * p.q_bs + h * p.q_hs + (size_t)min(qi, N - 1) * p.q_rs, g,
-              p.scale_log2, qi < N);
+    const bool low = split_row(qf[0], static_cast<const float *>(p.q) + b * p.q_bs + h * p.q_hs + (size_t)min(qi, N - 1) * p.q_rs,
+                               g, p.scale_log2 * kPartDown, qi < N);
     f32x4 acc[XT];
 #pragma unroll
     for (int xt = 0; xt < XT; ++xt) acc[xt] = zero4();
@@ -839,6 +839,7 @@ __device__ __forceinline__ void fwd_split_entry(const Params &p) {
     // a row with keys here whose first stage's scores all overflowed to -inf: m
     // stayed there, and O and the sum hold the later stages relative to 0
     if (m == -INFINITY && s_lo < s_hi && (!CAUSAL || s_lo * BK <= pos0 + qi)) z = NAN;
+    if (low) z = NAN;
     if (any_nonfinite<NW>(z, sm.flags, wave, lane)) {
         fwd_plain<NW, CAUSAL, PAGED, SPLIT>(p, bh, qb, s_lo * BK, s_hi * BK);
     } else if (qi < N) {
@@ -846,11 +847,11 @@ __device__ __forceinline__ void fwd_split_entry(const Params &p) {
             const size_t rows = (size_t)gridDim.z * p.B * p.Hq * N;
             const size_t r0 = ((size_t)blockIdx.z * p.B * p.Hq + bh) * N + qi;
 #pragma unroll
-            for (int xt = 0; xt < XT; ++xt) store4<float>(p.fwd_part + r0 * D + 16 * xt + 4 * g, acc[xt], 1.0f);
+            for (int xt = 0; xt < XT; ++xt) store4<float>(p.fwd_part + r0 * D + 16 * xt + 4 * g, acc[xt], kPartDown);
             if (g == 0) *reinterpret_cast<float2 *>(p.fwd_part + rows * D + 2 * r0) = make_float2(m, ltot);
         } else {
             float *O = static_cast<float *>(p.o) + b * p.o_bs + h * p.o_hs + (size_t)qi * p.o_rs;
-            const float inv = 1.0f / ltot;
+            const float inv = kPartDown / ltot;
 #pragma unroll
             for (int xt = 0; xt < XT; ++xt) store4<float>(O + 16 * xt + 4 * g, acc[xt], inv);
             if (p.lse != nullptr && g == 0) p.lse[(size_t)bh * N + qi] = (m + fast_log2(ltot)) * kLn2;

@@ -229,3 +229,44 @@ def test_chunk_split_over_128_query_blocks(n, nh, nkv, pos0):
         mx.run_prefill_paged(tq, tkp, tvp, b, tt, 16, pos0, nh, nkv, split=True, workspace=ws)
         assert torch.equal(a, b)
         assert _close(a.cpu().numpy(), want)
+
+
+@pytest.fixture(params=[True, False], ids=["one launch", "two launches"])
+def launches(request):
+    import mx230_amd as mx
+    old = mx.set_bwd_options(one_launch=request.param)
+    yield
+    mx.set_bwd_options(**old)
+
+
+@pytest.mark.parametrize("which", ["v", "do"])
+def test_small_values_keep_their_bits(launches, which):
+    """V or dO times 2^-100: O, dQ and dK (dV with dO) are those of the unscaled
+    operand times 2^-100, bit for bit (no normal fp32 value is held in fewer
+    bits), but for what cancels to the size of the smallest normals."""
+    rng = np.random.default_rng(3)
+    x = {n: (rng.uniform(0.5, 1.5, (3, 200, 64)) * rng.choice((-1, 1), (3, 200, 64))).astype(np.float32)
+         for n in ("q", "k", "v", "do")}
+    y = dict(x)
+    y[which] = np.ldexp(x[which], -100)
+    for causal in (False, True):
+        a, b = ([_fwd(z["q"], z["k"], z["v"], causal)[0], *_bwd(z["q"], z["k"], z["v"], z["do"], causal)] for z in (x, y))
+        for i, (got, want) in enumerate(zip(b, a)):
+            scaled = i in ((0, 1, 2) if which == "v" else (1, 2, 3))
+            want = np.ldexp(want, -100) if scaled else want
+            normal = np.abs(want) >= 2.0 ** -118
+            assert normal.mean() > 0.98 and np.array_equal(got[normal], want[normal]), (causal, i)
+            assert np.abs(got[~normal] - want[~normal]).max(initial=0) <= 2.0 ** -126, (causal, i)
+
+
+# the relative error (2-norm) is 3e-7 to 5e-7 at every size: 16 roundings of 2^-24
+@pytest.mark.parametrize("sizes", [(-118, 118, 0, 0), (118, -118, 0, 0), (-10, 10, -52, -52), (0, 0, -118, 0),
+                                   (0, 0, 0, -118)], ids=str)
+def test_small_against_large(launches, sizes):
+    """Q, K, V and dO of sizes 2^sizes whose scores are ordinary ones."""
+    rng = np.random.default_rng(4)
+    q, k, v, do = (np.ldexp(rng.standard_normal((2, 200, 64)).astype(np.float32), e) for e in sizes)
+    got = [_fwd(q, k, v, True)[0], *_bwd(q, k, v, do, True)]
+    for x, want in zip(got, [_ref(q, k, v, True)[0], *_ref_bwd(q, k, v, do, True)]):
+        c = np.abs(want).max()
+        assert np.linalg.norm((x - want) / c) <= 16 * 2.0 ** -24 * np.linalg.norm(want / c)
