@@ -182,10 +182,10 @@ int mxfa_run_bwd(const mxfa_shape *shape, const void *q, const void *k, const vo
  * mxfa_bwd_options.one_launch = 0 selects two launches, and so does a stream
  * under graph capture (a replayed launch would reuse the capture's flag
  * epoch); this query answers for an ordinary stream. An fp32 grid that fits the
- * GPU about at once also takes one launch unless one_launch = 0 (the dK/dV
- * work-groups compute Delta themselves, with no flags, captured or not; dK
- * and dV then equal the two launches' to fp32 rounding of Delta); this query
- * is 0 for it.
+ * GPU about at once also takes one launch unless one_launch = 0 or an output
+ * shares memory with an input (the dK/dV work-groups compute Delta themselves,
+ * with no flags, captured or not; dK and dV then equal the two launches' to
+ * fp32 rounding of Delta); this query is 0 for it.
  * No counterpart in the reference: it tells callers (and benchmarks) which
  * kernels the backward from O (main.rs:126-143, :179-210) becomes. */
 int mxfa_bwd_one_launch(const mxfa_shape *shape);

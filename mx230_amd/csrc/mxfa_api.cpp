@@ -262,6 +262,29 @@ int mxfa_run_bwd(const mxfa_shape *shape, const void *q, const void *k, const vo
     return mxfa_run_bwd_ws(shape, q, k, v, o, dout, lse, delta, dq, dk, dv, nullptr, 0, stream);
 }
 
+namespace {
+// True if dQ, dK, dV or the workspace shares memory with Q, K, V, O or dO. Two
+// launches allow some of it (dQ over O, dK over K, dV over V: each is last read
+// by the work-group or the launch before that writes it); in one launch other
+// work-groups still read what is written.
+bool bwd_in_place(const mxfa_shape *s, const Params &p, size_t workspace_bytes) {
+    const size_t row = (size_t)s->N * s->d * (s->dtype == MXFA_BF16 ? 2 : 4);
+    const size_t nq = (size_t)s->B * s->Hq * row, nk = (size_t)s->B * s->Hkv * row;
+    const struct {
+        const void *at;
+        size_t n;
+    } out[] = {{p.dq, nq}, {p.dk, nk}, {p.dv, nk}, {p.dkv_ws, p.dkv_ws != nullptr ? workspace_bytes : 0}},
+      in[] = {{p.q, nq}, {p.k, nk}, {p.v, nk}, {p.o_in, nq}, {p.dout, nq}};
+    for (const auto &x : out) {
+        for (const auto &y : in) {
+            const uintptr_t a = reinterpret_cast<uintptr_t>(x.at), b = reinterpret_cast<uintptr_t>(y.at);
+            if (a < b + y.n && b < a + x.n) return true;
+        }
+    }
+    return false;
+}
+}  // namespace
+
 int mxfa_run_bwd_ws(const mxfa_shape *shape, const void *q, const void *k, const void *v, const void *o,
                     const void *dout, const float *lse, float *delta, void *dq, void *dk, void *dv,
                     void *workspace, size_t workspace_bytes, void *stream) {
@@ -279,7 +302,8 @@ int mxfa_run_bwd_ws(const mxfa_shape *shape, const void *q, const void *k, const
         p.dk = dk;
         p.dv = dv;
         p.dkv_ws = static_cast<float *>(workspace);
-        if (mxfa::bwd_f32_together(p, shape->dtype == MXFA_BF16, shape->d, shape->causal))
+        if (mxfa::bwd_f32_together(p, shape->dtype == MXFA_BF16, shape->d, shape->causal) &&
+            !bwd_in_place(shape, p, workspace_bytes))
             return from_hip(mxfa::launch_bwd_f32(p, shape->causal, static_cast<hipStream_t>(stream)));
         if (mxfa::bwd_fused_available(p, shape->dtype == MXFA_BF16, shape->d, static_cast<hipStream_t>(stream))) {
             return from_hip(mxfa::launch_bwd_fused(p, shape->d, shape->causal, static_cast<hipStream_t>(stream)));

@@ -270,3 +270,27 @@ def test_small_against_large(launches, sizes):
     for x, want in zip(got, [_ref(q, k, v, True)[0], *_ref_bwd(q, k, v, do, True)]):
         c = np.abs(want).max()
         assert np.linalg.norm((x - want) / c) <= 16 * 2.0 ** -24 * np.linalg.norm(want / c)
+
+
+@pytest.mark.parametrize("Hkv", [4, 2], ids=["mha", "gqa"])
+def test_backward_in_place(launches, Hkv):
+    """dQ over O's memory, and dK and dV over K's and V's: the results of
+    separate outputs (a call whose outputs share memory with its inputs keeps
+    the two launches, between which those are no longer read)."""
+    import torch
+    import mx230_amd as mx
+    torch.manual_seed(8)
+    q, do = (torch.randn(2, 4, 300, 64, device="cuda") for _ in range(2))
+    k, v = (torch.randn(2, Hkv, 300, 64, device="cuda") for _ in range(2))
+    o, lse = mx.attention_fwd(q, k, v, True)
+    delta = torch.empty_like(lse)
+    old = mx.set_bwd_options(one_launch=False)
+    dq, dk, dv = (torch.empty_like(x) for x in (q, k, v))
+    mx.run_bwd(q, k, v, o, do, lse, delta, dq, dk, dv, True)
+    mx.set_bwd_options(**old)
+    o2 = o.clone()
+    mx.run_bwd(q, k, v, o2, do, lse, delta, o2, dk2 := torch.empty_like(k), dv2 := torch.empty_like(v), True)
+    assert torch.equal(o2, dq) and torch.equal(dk2, dk) and torch.equal(dv2, dv)
+    k2, v2, dq2 = k.clone(), v.clone(), torch.empty_like(q)
+    mx.run_bwd(q, k2, v2, o, do, lse, delta, dq2, k2, v2, True)
+    assert torch.equal(dq2, dq) and torch.equal(k2, dk) and torch.equal(v2, dv)
