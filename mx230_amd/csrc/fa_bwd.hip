@@ -1511,14 +1511,18 @@ __device__ __forceinline__ void dkv_split_body(const Params &p, const DkvWork wk
     const float kmul = part ? 1.0f : -p.scale;
     float z = low ? NAN : 0.f;
 #pragma unroll
-    for (int xt = 0; xt < XT; ++xt) z += zero_of(accK[xt]) + zero_of(accV[xt]);
+    for (int xt = 0; xt < XT; ++xt) {
+        accK[xt] *= kDsDown * kPartDown;
+        accV[xt] *= kPartDown;
+        z += zero_of(accK[xt]) + zero_of(accV[xt]);
+    }
     if (any_nonfinite<4>(z, sm.flags, wave, lane)) {
         dkv_plain<CAUSAL, OWN>(p, wk.bkv, wk.kb, g0, nsteps, dK, dV, kmul);
     } else if (key < N) {
 #pragma unroll
         for (int xt = 0; xt < XT; ++xt) {
-            store4<float>(dK + (size_t)key * D + 16 * xt + 4 * g, accK[xt] * (kDsDown * kPartDown), kmul);
-            store4<float>(dV + (size_t)key * D + 16 * xt + 4 * g, accV[xt], kPartDown);
+            store4<float>(dK + (size_t)key * D + 16 * xt + 4 * g, accK[xt], kmul);
+            store4<float>(dV + (size_t)key * D + 16 * xt + 4 * g, accV[xt], 1.0f);
         }
     }
     wg_time_after_stores();
