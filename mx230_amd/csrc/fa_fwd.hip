@@ -1135,18 +1135,32 @@ static hipError_t launch_fwd_f32(Params p, int causal, hipStream_t stream) {
     return launch_kernel(id, grid, dim3(64 * nw), args, stream);
 }
 
-// Few query rows of a prefill: fwd_few_entry, unsplit at any number of keys (one
-// token, us a call: 8/1 heads d = 128 after 2000 positions 27.2 -> 17.1, 14/2
-// heads after 65535 555 -> 370, 32/32 heads after 8191 paged 78 -> 70), and
-// split where the 256 work-groups that fit at once (8 waves; d = 128: 4) leave
-// each wave at most two stages. Beyond that the 64-query form's work-groups,
-// whose waves load each tile together, read faster: 14/2 heads after 65535
-// 24.6 -> 13.1, 8/8 after 20000 17.4 -> 13.5, but 32/8 after 65535 26.5
-// against 30.9, and d = 128 45 against 50.
-static bool fwd_few(const Params &p, int dtype_bf16) { return dtype_bf16 && p.prefill != 0 && p.N <= kFewRows; }
+// Few query rows of a prefill, unsplit (bh rows' blocks; the same rule for a
+// paged cache, so that both give the same bits). fwd_few_entry's work-groups
+// take a CU each:
+//  * more than 256 of them run in rounds, where the 64-query form holds two or
+//    three a CU (8 tokens, d = 64, 16 stages: 288 heads 1.3 times its time, 512
+//    1.3, 256 1.16), and with one stage nothing is gained (3.9 -> 4.2 us);
+//  * up to one stage per wave of all 256 (8 waves; d = 128: 4) they read faster:
+//    us, 8 tokens, 128 heads of 16 stages 0.76 times, 8 heads of 125 0.51;
+//  * beyond that the caches set the time: as fast up to 192 blocks at d = 64
+//    (0.94-1.04; paged 0.83-0.97; 256: 1.25), and at d = 128 up to 64 (0.90;
+//    96 and 128 0.94-1.12, 160 1.08-1.17).
+static bool few_rows(const Params &p, int dtype_bf16) { return dtype_bf16 && p.prefill != 0 && p.N <= kFewRows; }
+static long long key_stages(const Params &p) { return (std::min(p.Nk, p.pos0 + p.N) + 63) / 64; }
+static bool fwd_few(const Params &p, int dtype_bf16, int d) {
+    const long long stages = key_stages(p), bh = (long long)p.B * p.Hq;
+    return few_rows(p, dtype_bf16) && stages > 1 && bh <= 256 &&
+           (bh * stages <= 256 * (d == 128 ? 4 : 8) || bh <= (d == 128 ? 64 : 192));
+}
+// Split: up to 7/8 of a stage per wave of the 256 work-groups that fit at once
+// (0.72-1.0 times the 64-query form's time; at a whole one 0.9-1.11, and with
+// two 1.0-1.2 at d = 64); below 8 blocks, which the 64-query form splits into
+// fewer work-groups than CUs, up to two stages (one token, 1 to 7 heads, d = 64:
+// 0.26-0.89 times).
 static bool fwd_few_split(const Params &p, int dtype_bf16, int d) {
-    const long long stages = (std::min(p.Nk, p.pos0 + p.N) + 63) / 64;
-    return fwd_few(p, dtype_bf16) && (long long)p.B * p.Hq * stages <= 2 * 256 * (d == 128 ? 4 : 8);
+    const long long bh = (long long)p.B * p.Hq, waves = 256 * (d == 128 ? 4 : 8);
+    return few_rows(p, dtype_bf16) && bh * key_stages(p) <= (bh < 8 ? 2 * waves : waves / 8 * 7);
 }
 
 static hipError_t launch_fwd_few(const Params &p, int d, int splits, hipStream_t stream) {
@@ -1169,7 +1183,7 @@ static int fwd_splits_64(const Params &p, int dtype_bf16, int d, long long most)
     const long long wgs = (long long)p.B * p.Hq * ((p.N + 63) / 64);
     const long long slots = 256LL * (dtype_bf16 && d == 64 ? 3 : 2);
     if (2 * wgs >= slots) return 1;
-    const long long stages = (std::min(p.Nk, p.pos0 + p.N) + 63) / 64;  // the heaviest block's
+    const long long stages = key_stages(p);  // the heaviest block's
     if (stages < (dtype_bf16 ? 16 : 8)) return 1;
     return (int)std::min({(slots + wgs - 1) / wgs, std::max(1LL, stages / 2), most});
 }
@@ -1182,7 +1196,7 @@ static int fwd_splits_64(const Params &p, int dtype_bf16, int d, long long most)
 // 13.5 against 15.6.
 static bool fwd_f32_wide(const Params &p, int dtype_bf16) {
     if (dtype_bf16 || p.N <= 64) return false;
-    const long long stages = (std::min(p.Nk, p.pos0 + p.N) + 63) / 64, bh = (long long)p.B * p.Hq;
+    const long long stages = key_stages(p), bh = (long long)p.B * p.Hq;
     return stages >= 16 && bh * ((p.N + 127) / 128) < 256 &&
            bh * ((p.N + 63) / 64) * std::min(stages / 2, (long long)kFwdMaxSplits) >= 512;
 }
@@ -1190,7 +1204,7 @@ static bool fwd_f32_wide(const Params &p, int dtype_bf16) {
 // The forms that split into one round of the work-groups that fit at once:
 // those, and fwd_few_entry's 256; else fwd_splits_64's.
 int fwd_splits(const Params &p, int dtype_bf16, int d) {
-    const long long stages = (std::min(p.Nk, p.pos0 + p.N) + 63) / 64, bh = (long long)p.B * p.Hq;
+    const long long stages = key_stages(p), bh = (long long)p.B * p.Hq;
     if (fwd_f32_wide(p, dtype_bf16))
         return (int)std::min({512 / (bh * ((p.N + 127) / 128)), stages / 2, (long long)kFwdMaxSplits});
     const bool few = fwd_few_split(p, dtype_bf16, d);
@@ -1200,7 +1214,7 @@ int fwd_splits(const Params &p, int dtype_bf16, int d) {
 
 int fwd_splits_in(const Params &p, int dtype_bf16, int d, size_t bytes) {
     const int want = fwd_splits(p, dtype_bf16, d), must = fwd_splits_64(p, dtype_bf16, d, kFwdMaxSplits);
-    if (want <= 1) return 1;  // few rows of more than 128 heads: unsplit, where 64-query work-groups split
+    if (want <= 1) return 1;  // no workspace is reported for it, so none is asked for
     const size_t one = (size_t)p.B * p.Hq * p.N * (size_t)(d + 2) * sizeof(float);
     const int fit = (int)std::min<size_t>(bytes / one, (size_t)want);
     if (must <= 1) return std::max(fit, 1);
@@ -1241,7 +1255,7 @@ hipError_t launch_fwd_split(const Params &p, int dtype_bf16, int d, int splits, 
 
 hipError_t launch_fwd(const Params &p, int dtype_bf16, int d, int causal, hipStream_t stream) {
     if (p.block_table != nullptr && !causal) return hipErrorInvalidValue;  // paged kernels are causal
-    if (causal && fwd_few(p, dtype_bf16)) return launch_fwd_few(p, d, 1, stream);
+    if (causal && fwd_few(p, dtype_bf16, d)) return launch_fwd_few(p, d, 1, stream);
     if (!dtype_bf16) return d == 64 ? launch_fwd_f32(p, causal, stream) : hipErrorInvalidValue;
     if (d == 64) return causal ? launch_fwd_t<PolBF16<64>, true>(p, stream) : launch_fwd_t<PolBF16<64>, false>(p, stream);
     if (d == 128)

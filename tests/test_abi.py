@@ -261,6 +261,9 @@ def test_prefill_paged_null_and_alignment(lib):
     (dict(n_tok=4096, pos0=0), 1),                 # 896 work-groups fill the GPU
     (dict(n_tok=960, pos0=100, n_head=1, n_kv_head=1, q_stride=3 * 64, kv_stride=64, out_stride=64), 8),
     (dict(n_tok=100, pos0=100000, n_head=1, n_kv_head=1, q_stride=3 * 64, kv_stride=64, out_stride=64), 32),
+    # one row of many heads: 64-query work-groups from more than 7/8 of a stage per few-row wave on
+    (dict(n_tok=1, pos0=1100, n_head=96, n_kv_head=96, q_stride=288 * 64, kv_stride=96 * 64, out_stride=96 * 64), 2),
+    (dict(n_tok=1, pos0=1500, n_head=96, n_kv_head=96, q_stride=288 * 64, kv_stride=96 * 64, out_stride=96 * 64), 8),
 ])
 def test_prefill_split_workspace(lib, kw, splits):
     """The split prefill's workspace: splits x rows x (head_dim + 2) fp32, 0 when no split pays."""

@@ -19,8 +19,9 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("n,nh,nkv,pos0", [
     (1, 1, 1, 0), (1, 7, 1, 62), (1, 7, 1, 63), (1, 16, 1, 64), (1, 8, 2, 511), (1, 8, 2, 512), (1, 4, 4, 1023),
     (1, 14, 2, 1024), (1, 8, 1, 8200), (1, 3, 1, 40000), (16, 2, 1, 100), (16, 2, 1, 1500), (3, 4, 2, 0), (5, 2, 2, 1021),
-    # more than 128 heads of rows: unsplit with any workspace or none
-    (1, 144, 144, 1200), (8, 144, 12, 1200)])
+    # around the ends of the few-row kernels' range: one stage, 192, 256 and more heads,
+    # more stages than its waves hold at once
+    (1, 144, 144, 1200), (8, 144, 12, 1200), (2, 192, 96, 700), (16, 256, 64, 120), (2, 257, 257, 100), (1, 64, 64, 4100)])
 def test_few_rows(n, nh, nkv, pos0, hd):
     import torch
     import mx230_amd as mx
