@@ -863,16 +863,23 @@ __device__ __forceinline__ void fwd_split_entry(const Params &p) {
 // Adds the S key splits of a split forward (fwd_entry<..., SPLIT>): with M the
 // largest of the splits' running maxima (log2 units), O = sum_s 2^(m_s - M)
 // O_s / sum_s 2^(m_s - M) l_s, written as the forward writes O. A split that
-// holds no key of the row has m = -inf and weight 0. Up to kMergeThread splits
-// (many rows then): one thread per four elements of a row, every split's loads
-// issued before the first is used, so a call costs one memory latency. More
-// splits (few rows): a work-group per row, its groups of threads over the
-// (fwd_merge_row_body): with a thread per four elements one token's 32 rows
-// are two work-groups, each reading 131 KB (32 splits 4.7 -> 3.1 us; the
-// 128 splits of 14 rows 3.6).
+// holds no key of the row has m = -inf and weight 0. Two forms:
+//  * one thread per four elements of a row, every split's loads issued before
+//    the first is used, so a call costs one memory latency (fwd_merge_body;
+//    MAXS = 8 keeps the registers of the common case low, the 32-split form
+//    takes 205): up to kMergeThread splits, and more with many rows;
+//  * a work-group per row, its groups of threads over the splits
+//    (fwd_merge_row_body), for more splits of at most kMergeRow elements of O:
+//    with a thread per four elements one token's 32 rows are two work-groups, each
+//    reading 131 KB (32 splits 4.7 -> 3.1 us; the 128 splits of 14 rows 3.6).
+// The line, us a call, a work-group per row against a thread per four elements:
+// d = 64, 1000 rows of 12 splits 9.5 / 9.9 and of 32 16.2 / 17.2, 1200 of 10 9.7 /
+// 9.9, 1400 of 9 10.3 / 10.1, 4000 of 12 17.8 / 16.7, 7000 of 9 (fp32) 40.7 / 39.1;
+// d = 128, 400 of 32 13.1 / 14.4, 1000 of 32 19.6 / 19.5, 3600 of 9 24.0 / 23.0.
 constexpr int kFwdMaxSplits = 32;   // of 64-query work-groups
 constexpr int kFewMaxSplits = 128;  // of fwd_few_entry's
 constexpr int kMergeThread = 8;
+constexpr size_t kMergeRow = 1 << 16;
 
 template <class T, int D, int MAXS>
 __device__ __forceinline__ void fwd_merge_body(const Params &p, int S) {
@@ -1030,6 +1037,9 @@ MXFA_FWD_SP(mxfa_fwd_b128_c_w2_q1_pg_sp, PolBF16<128>, 2, true)
 MXFA_FWD_MERGE(mxfa_fwd_merge8_b64, u16, 64, kMergeThread)
 MXFA_FWD_MERGE(mxfa_fwd_merge8_b128, u16, 128, kMergeThread)
 MXFA_FWD_MERGE(mxfa_fwd_merge8_f64, float, 64, kMergeThread)
+MXFA_FWD_MERGE(mxfa_fwd_merge32t_b64, u16, 64, kFwdMaxSplits)
+MXFA_FWD_MERGE(mxfa_fwd_merge32t_b128, u16, 128, kFwdMaxSplits)
+MXFA_FWD_MERGE(mxfa_fwd_merge32t_f64, float, 64, kFwdMaxSplits)
 #define MXFA_FWD_MERGE_ROW(NAME, T, D, MAXS)                                                           \
     extern "C" __global__ __launch_bounds__(8 * MAXS) void NAME(Params p, int splits) {                \
         fwd_merge_row_body<T, D, MAXS>(p, splits);                                                     \
@@ -1235,22 +1245,23 @@ hipError_t launch_fwd_split(const Params &p, int dtype_bf16, int d, int splits, 
                               : (pg ? k_mxfa_fwd_b128_c_w2_q1_pg_sp : k_mxfa_fwd_b128_c_w2_q1_sp))
         : nw == 8  ? (pg ? k_mxfa_fwd_f64_c_pg_sp_g8 : k_mxfa_fwd_f64_c_sp_g8)
                    : (pg ? k_mxfa_fwd_f64_c_pg_sp : k_mxfa_fwd_f64_c_sp);
-    const int mi = splits <= kMergeThread ? 0 : splits <= kFwdMaxSplits ? 1 : 2;  // 2: few rows, bf16
-    static constexpr KernelId merge[3][3] = {
-        {k_mxfa_fwd_merge8_b64, k_mxfa_fwd_merge32_b64, k_mxfa_fwd_merge128_b64},
-        {k_mxfa_fwd_merge8_b128, k_mxfa_fwd_merge32_b128, k_mxfa_fwd_merge128_b128},
-        {k_mxfa_fwd_merge8_f64, k_mxfa_fwd_merge32_f64, k_mxfa_fwd_merge32_f64}};
+    const size_t rows = (size_t)p.B * p.Hq * p.N;
+    // 0, 1: a thread per four elements; 2, 3: a work-group per row (3: few rows, bf16)
+    const int mi = splits <= kMergeThread ? 0 : splits > kFwdMaxSplits ? 3 : rows * d > kMergeRow ? 1 : 2;
+    static constexpr KernelId merge[3][4] = {
+        {k_mxfa_fwd_merge8_b64, k_mxfa_fwd_merge32t_b64, k_mxfa_fwd_merge32_b64, k_mxfa_fwd_merge128_b64},
+        {k_mxfa_fwd_merge8_b128, k_mxfa_fwd_merge32t_b128, k_mxfa_fwd_merge32_b128, k_mxfa_fwd_merge128_b128},
+        {k_mxfa_fwd_merge8_f64, k_mxfa_fwd_merge32t_f64, k_mxfa_fwd_merge32_f64, k_mxfa_fwd_merge32_f64}};
     const KernelId km = merge[!dtype_bf16 ? 2 : d == 128 ? 1 : 0][mi];
     Params q = p;
     void *args[] = {&q};
     hipError_t e = few ? launch_fwd_few(p, d, splits, stream)
                        : launch_kernel(kf, dim3(p.B * p.Hq, (p.N + 16 * nw - 1) / (16 * nw), splits), dim3(64 * nw), args, stream);
     if (e != hipSuccess) return e;
-    const size_t rows = (size_t)p.B * p.Hq * p.N;
     int s = splits;
     void *margs[] = {&q, &s};
-    const unsigned groups = (unsigned)(mi == 0 ? (rows * (d / 4) + 255) / 256 : rows);
-    return launch_kernel(km, dim3(groups), dim3(mi == 2 ? 8 * kFewMaxSplits : 256), margs, stream);
+    const unsigned groups = (unsigned)(mi <= 1 ? (rows * (d / 4) + 255) / 256 : rows);
+    return launch_kernel(km, dim3(groups), dim3(mi == 3 ? 8 * kFewMaxSplits : 256), margs, stream);
 }
 
 hipError_t launch_fwd(const Params &p, int dtype_bf16, int d, int causal, hipStream_t stream) {

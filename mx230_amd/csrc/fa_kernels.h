@@ -25,6 +25,7 @@
     X(mxfa_fwd_b64_c_w3_q1_pg_sp) X(mxfa_fwd_b128_c_w2_q1_pg_sp) X(mxfa_fwd_f64_c_pg_sp)       \
     X(mxfa_fwd_merge8_b64) X(mxfa_fwd_merge8_b128) X(mxfa_fwd_merge8_f64)                     \
     X(mxfa_fwd_merge32_b64) X(mxfa_fwd_merge32_b128) X(mxfa_fwd_merge32_f64)                  \
+    X(mxfa_fwd_merge32t_b64) X(mxfa_fwd_merge32t_b128) X(mxfa_fwd_merge32t_f64)               \
     X(mxfa_fwd_merge128_b64) X(mxfa_fwd_merge128_b128)                                        \
     X(mxfa_fwd_b64_few) X(mxfa_fwd_b64_few_pg) X(mxfa_fwd_b64_few_sp) X(mxfa_fwd_b64_few_pg_sp) \
     X(mxfa_fwd_b128_few) X(mxfa_fwd_b128_few_pg) X(mxfa_fwd_b128_few_sp) X(mxfa_fwd_b128_few_pg_sp) \

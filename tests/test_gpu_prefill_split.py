@@ -140,3 +140,15 @@ def test_split_workspace_reuse_and_size():
     assert rel_err(small_out.float().cpu().numpy(), out[:200].float().cpu().numpy()) <= TOL_BF16
     with pytest.raises(mx.MxfaError):
         mx.run_prefill_split(tq, tk, tv, out, 3584, 14, 2, 64, workspace=ws[:ws.numel() - 16])
+
+
+@pytest.mark.parametrize("hd,bf16", [(64, True), (128, True), (64, False)])
+@pytest.mark.parametrize("more", [0, 1])
+def test_merge_forms(more, hd, bf16):
+    """More than 8 splits on both sides of the size of O (2^16 elements) from
+    which the merge takes a thread per four elements."""
+    n_tok = 2 ** 16 // (8 * hd) + more
+    import mx230_amd as mx
+    splits = mx.prefill_workspace_bytes(n_tok, 2000, 8, 2, hd, bf16) // (8 * n_tok * (hd + 2) * 4)
+    assert 8 < splits <= 32
+    _run(n_tok=n_tok, pos0=2000, nh=8, nkv=2, hd=hd, bf16=bf16, seed=20)
