@@ -1132,11 +1132,15 @@ static hipError_t launch_fwd_t(const Params &p, hipStream_t stream) {
 // two that a CU holds (each K and V element is then split half as often: B4 H12
 // N4096 causal 590 -> 523 us); 4 waves and 64 queries on smaller grids (B4 H12
 // N1024 causal 60 -> 54, B1 H1 N256 16.8 -> 14.1; 384 of 128 queries, B1 H12
-// N4096, 310 and 318 non-causal, 192 both causal). The same waves, so the
-// same bits.
+// N4096, 310 and 318 non-causal, 192 both causal). A last block of 128 with at
+// most 64 rows leaves half its waves idle, which costs more than that saves in
+// heads of 1, 3 or 5 blocks of 64 (512 heads of 64 rows 9.5 us against 11.2, of
+// 192 32.0 / 37.5, of 320 64.7 / 69.1; of 256 46.6 / 43.9). The same waves, so
+// the same bits.
 static hipError_t launch_fwd_f32(Params p, int causal, hipStream_t stream) {
     const bool pg = p.block_table != nullptr;
-    const int nw = (long long)p.B * p.Hq * ((p.N + 127) / 128) >= 512 ? 8 : 4;
+    const int nb64 = (p.N + 63) / 64;
+    const int nw = (long long)p.B * p.Hq * ((p.N + 127) / 128) >= 512 && (nb64 % 2 == 0 || nb64 > 5) ? 8 : 4;
     const dim3 grid(p.B * p.Hq, (p.N + 16 * nw - 1) / (16 * nw));
     const KernelId id = nw == 8 ? (pg ? k_mxfa_fwd_f64_c_pg_g8 : causal ? k_mxfa_fwd_f64_c_g8 : k_mxfa_fwd_f64_n_g8)
                                 : (pg ? k_mxfa_fwd_f64_c_pg : causal ? k_mxfa_fwd_f64_c : k_mxfa_fwd_f64_n);

@@ -49,7 +49,7 @@ def _close(got, want):
 # remainder of the 16-, 32-, 64- and 128-row tiles
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("H,Hkv,N", [(1, 1, 1), (1, 1, 31), (2, 1, 33), (1, 1, 64), (3, 3, 65), (4, 2, 129),
-                                     (33, 11, 511), (512, 64, 100)])
+                                     (33, 11, 511), (512, 64, 100), (512, 64, 33), (256, 32, 150)])
 def test_forward_edges(H, Hkv, N, causal):
     rng = np.random.default_rng(H * 1000 + N)
     q, k, v = (rng.standard_normal((h, N, 64)).astype(np.float32) for h in (H, Hkv, Hkv))
