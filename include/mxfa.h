@@ -184,8 +184,8 @@ int mxfa_run_bwd(const mxfa_shape *shape, const void *q, const void *k, const vo
  * epoch); this query answers for an ordinary stream. An fp32 grid that fits the
  * GPU about at once also takes one launch unless one_launch = 0 or an output
  * shares memory with an input (the dK/dV work-groups compute Delta themselves,
- * with no flags, captured or not; dK and dV then equal the two launches' to
- * fp32 rounding of Delta); this query is 0 for it.
+ * in the dQ work's order, with no flags, captured or not, so the results equal
+ * the two launches' bitwise); this query is 0 for it.
  * No counterpart in the reference: it tells callers (and benchmarks) which
  * kernels the backward from O (main.rs:126-143, :179-210) becomes. */
 int mxfa_bwd_one_launch(const mxfa_shape *shape);

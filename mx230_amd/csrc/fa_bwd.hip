@@ -1195,11 +1195,13 @@ __device__ __forceinline__ void dkv_plain(const Params &p, int bkv, int kb, int 
             const float *Q = static_cast<const float *>(p.q) + r * D + c;
             const float *G = static_cast<const float *>(p.dout) + r * D + c;
             float delta;
-            if constexpr (OWN) {
+            if constexpr (OWN) {  // in dq_split_body's order
+                const float *g1 = static_cast<const float *>(p.dout) + r * D + c / 2;
+                const float *o1 = static_cast<const float *>(p.o_in) + r * D + c / 2;
                 delta = 0.f;
 #pragma unroll
                 for (int e = 0; e < 16; ++e)
-                    delta = __builtin_fmaf(G[e], static_cast<const float *>(p.o_in)[r * D + c + e], delta);
+                    delta = __builtin_fmaf(g1[32 * (e >> 3) + (e & 7)], o1[32 * (e >> 3) + (e & 7)], delta);
                 delta = quad_sum(delta);
             } else {
                 delta = p.delta[r];
@@ -1269,7 +1271,7 @@ __device__ __forceinline__ void dq_split_body(const Params &p, int bh, int qb, B
             const int c = 32 * (e >> 3) + 8 * g + (e & 7);
             dl = __builtin_fmaf(d[c], o[c], dl);
         }
-        dl = xg_sum(dl);
+        dl = xg_sum_pairs(dl);
         if (qi < N && g == 0) p.delta[qrow] = dl;
     } else {
         dl = p.delta[qrow];
@@ -1479,16 +1481,13 @@ __device__ __forceinline__ void dkv_split_body(const Params &p, const DkvWork wk
         xg.write(sm.b, tid);
         if (wave == 0) sm.sL[lane] = -xl * kLog2e;
         if constexpr (OWN) {
-            // a row's chunks: two of each lane pair, the pair's and those of the
-            // pair 128 threads on
+            // a row's chunks: two of each lane pair (c and c + 4), the pair's and
+            // those of the pair 128 threads on; summed as dq_split_body's lanes do
             float d = 0.f;
 #pragma unroll
             for (int k = 0; k < Stage::NK; ++k) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    d = __builtin_fmaf(xg.x[k][0][e], o[k][0][e], d);
-                    d = __builtin_fmaf(xg.x[k][1][e], o[k][1][e], d);
-                }
+                for (int e = 0; e < 8; ++e) d = __builtin_fmaf(xg.x[k][e >> 2][e & 3], o[k][e >> 2][e & 3], d);
             }
             d += __shfl_xor(d, 1, 64);
             if ((tid & 1) == 0) sm.sD[tid >> 7][srow[0]] = d * kDsUp;

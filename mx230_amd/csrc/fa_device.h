@@ -191,6 +191,15 @@ __device__ __forceinline__ float xg_sum(float x) {
     return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
+// The same sum as (g0 + g1) + (g2 + g3): the fp32 Delta, which the dK/dV work of
+// the one-launch backward computes in this order from its own layout.
+__device__ __forceinline__ float xg_sum_pairs(float x) {
+    auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+
 // Makes x opaque to the optimiser (an empty asm that "modifies" it), so a value
 // computed once before a loop is not recomputed inside it.
 template <class X>

@@ -294,3 +294,26 @@ def test_backward_in_place(launches, Hkv):
     k2, v2, dq2 = k.clone(), v.clone(), torch.empty_like(q)
     mx.run_bwd(q, k2, v2, o, do, lse, delta, dq2, k2, v2, True)
     assert torch.equal(dq2, dq) and torch.equal(k2, dk) and torch.equal(v2, dv)
+
+
+@pytest.mark.parametrize("Hkv,N,causal", [(4, 1, True), (4, 65, False), (2, 300, True), (1, 513, False)])
+@pytest.mark.parametrize("finite", [True, False])
+def test_one_launch_equals_two_launches(Hkv, N, causal, finite):
+    """The one-launch fp32 backward gives the two launches' bits, also where the
+    work-groups run again in plain fp32 (an infinite key element)."""
+    import torch
+    import mx230_amd as mx
+    torch.manual_seed(N)
+    q, do = (torch.randn(2, 4, N, 64, device="cuda") for _ in range(2))
+    k, v = (torch.randn(2, Hkv, N, 64, device="cuda") for _ in range(2))
+    if not finite:
+        q[..., 0] = -q[..., 0].abs() - 0.1
+        k[:, :, N // 2, 0] = float("inf")
+    o, lse = mx.attention_fwd(q, k, v, causal)
+    res = []
+    for one in (True, False):
+        old = mx.set_bwd_options(one_launch=one)
+        res.append(mx.attention_bwd(q, k, v, o, lse, do, causal))
+        mx.set_bwd_options(**old)
+    for a, b in zip(*res):
+        assert torch.equal(a.view(torch.int32), b.view(torch.int32))
