@@ -21,6 +21,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import warnings
 from dataclasses import dataclass
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -177,18 +178,34 @@ def load_library(path: str | None = None):
 _native = None
 
 
+class _NoBinding:
+    """In the place of csrc/binding.cpp where it cannot be loaded: leaves every
+    call to the Python path."""
+
+    @staticmethod
+    def _other(*args):
+        return NotImplemented
+    attention_fwd = attention_bwd = prefill = _other
+
+
 def _calls():
     """The call path in C++ (csrc/binding.cpp), bound to the loaded libmxfa: its
     functions take plain GPU tensors on torch's current stream and return
-    NotImplemented for every other call, which the Python below then takes."""
+    NotImplemented for every other call, which the Python below then takes.
+    Where the module is not built or cannot be loaded (another torch), it
+    warns once, and every call goes the Python way."""
     global _native
     if _native is None:
         lib = load_library()
+        _torch()  # whose libraries the module is linked with
         try:
             from . import _binding as ext
         except ImportError as e:
-            raise ImportError(f"{os.path.join(_HERE, '_binding.so')} cannot be loaded ({e}): build it with "
-                              "`make -C mx230_amd/csrc` (or __graft_entry__.build())") from e
+            warnings.warn(f"{os.path.join(_HERE, '_binding.so')} cannot be loaded ({e}); calls cost 10-30 us more on "
+                          "the host. Build it with `make -C mx230_amd/csrc` (or __graft_entry__.build())",
+                          RuntimeWarning, stacklevel=3)
+            _native = _NoBinding
+            return _native
         ext.bind(*(ctypes.cast(getattr(lib, f), ctypes.c_void_p).value for f in (
             "mxfa_run_flash_lse", "mxfa_run_bwd_ws", "mxfa_bwd_workspace_bytes", "mxfa_run_prefill",
             "mxfa_run_prefill_ws", "mxfa_run_prefill_paged", "mxfa_run_prefill_paged_ws")))

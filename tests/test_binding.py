@@ -3,6 +3,10 @@ GPU tensors only, and gives what the Python path (taken with an explicit
 stream) gives, bit for bit."""
 from __future__ import annotations
 
+import os
+import subprocess
+import sys
+
 import pytest
 
 import mx230_amd as mx
@@ -17,6 +21,31 @@ def test_leaves_other_calls_to_python():
     assert c.attention_bwd(q, q, q, q, q, q, True, 0.0) is NotImplemented
     assert c.prefill(q, q, q, q, None, 0, 0, 1, 1, 64, 0.0, False, None) is NotImplemented
     assert c.prefill() is NotImplemented
+
+
+def test_without_the_module(monkeypatch):
+    """Where _binding.so is missing or does not load, the package warns once and
+    takes the Python path."""
+    import torch
+    monkeypatch.setattr(mx, "_native", None)
+    monkeypatch.delattr(mx, "_binding", raising=False)
+    monkeypatch.setitem(sys.modules, "mx230_amd._binding", None)
+    with pytest.warns(RuntimeWarning, match="_binding.so"):
+        c = mx._calls()
+    assert c.prefill() is NotImplemented and mx._calls() is c
+    q = torch.zeros(1, 1, 4, 64)
+    with pytest.raises(ValueError, match="device tensor"):  # raised by the Python path
+        mx.attention_fwd(q, q, q, True)
+
+
+@pytest.mark.parametrize("python,built", [(sys.executable, True), ("/bin/false", False)])
+def test_make_without_torch(python, built):
+    """The C library's build needs no torch and no Python headers: where they are
+    missing the extension module is left out."""
+    r = subprocess.run(["make", "-n", "-B", "-C", os.path.join(os.path.dirname(mx.LIB_PATH), "csrc"),
+                        f"PYTHON={python}"], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    assert ("binding.cpp" in r.stdout) == built and "libmxfa.so" in r.stdout
 
 
 @pytest.mark.gpu
