@@ -1897,17 +1897,6 @@ static long long dkv_work_groups(const Params &p, bool causal, int BKV) {
     return n;
 }
 
-int dkv_split(const Params &p, int dtype_bf16, int d, int causal) {
-    Params q = p;
-    if (dtype_bf16) {
-        if (d == 64) dkv_plan_t<DkvB64>(q, causal != 0);
-        if (d == 128) dkv_plan_t<DkvB128>(q, causal != 0);
-    } else if (d == 64) {
-        dkv_plan_t<DkvF32>(q, causal != 0);
-    }
-    return q.dkv_split;
-}
-
 // Bytes of the fp32 partial planes of a split (p.dkv_split set): dK's planes,
 // then dV's.
 static size_t dkv_planes_bytes(const Params &p, int d) {

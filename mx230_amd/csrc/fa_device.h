@@ -253,14 +253,14 @@ struct PolBF16 {
     static constexpr int EPC = 8;      // elements per 16-byte chunk
     static constexpr int NC = D / 32;  // MFMAs over D per first-GEMM tile
     static constexpr int ROWS = 64;    // rows of every LDS tile
-    // waves per SIMD the forward (kWaves), dQ (kWavesDq) and dK/dV (kWavesDkv)
+    // waves per SIMD the forward (fa_fwd.hip), dQ (kWavesDq) and dK/dV (kWavesDkv)
     // kernels are compiled for: the largest count that fits without spills in
     // their loops. Three work-groups per CU also balance the causal passes:
     // their 128-row work-groups (64 - 2i stages of 64 for i = 0..31 at
-    // N = 4096) pair up into equal loads over 768 slots. The forward also has
-    // a three-wave form (kWavesFwdCausal) for causal launches of at least 768
-    // work-groups; on smaller causal grids and non-causal launches it is no
-    // faster than two. At d = 128 all three kernels run two waves per SIMD
+    // N = 4096) pair up into equal loads over 768 slots. The causal forward
+    // takes its 128-query form only from 768 work-groups on, three waves
+    // (kWavesFwdCausal); non-causal launches are no faster with three than
+    // with two. At d = 128 all three kernels run two waves per SIMD
     // (dK/dV is held there by its 66 KB of LDS; the non-causal forward spills
     // 64 bytes per lane at two and still ran 22% faster than at one).
     // The register-resident operand of each score GEMM (Q in the forward and
@@ -269,7 +269,6 @@ struct PolBF16 {
     // operand to bf16 instead puts an error of about |S log2(e)| 2^-9 into
     // every exponent, correlated along a row or a key, which grows with the
     // logits and reaches the outputs through LSE.
-    static constexpr int kWaves = 2;
     static constexpr int kWavesFwdCausal = D == 64 ? 3 : 2;
     static constexpr int kWavesDq = D == 64 ? 3 : 2;
     // dQ pass: 16-query tiles per wave and waves per work-group. 64 queries

@@ -993,7 +993,6 @@ __device__ __forceinline__ void fwd_merge_row_body(const Params &p, int S) {
 #define MXFA_FWD_PG(NAME, POL, WPS, QT)                                                                 \
     extern "C" __global__ __launch_bounds__(256, WPS) void NAME(Params p) { fwd_entry<POL, true, QT, true>(p); }
 MXFA_FWD(mxfa_fwd_b64_c_w3_q2, PolBF16<64>, true, 3, 2)
-MXFA_FWD(mxfa_fwd_b64_c_w2_q2, PolBF16<64>, true, 2, 2)
 MXFA_FWD(mxfa_fwd_b64_c_w3_q1, PolBF16<64>, true, 3, 1)
 MXFA_FWD(mxfa_fwd_b64_n_w2_q2, PolBF16<64>, false, 2, 2)
 MXFA_FWD(mxfa_fwd_b64_n_w3_q1, PolBF16<64>, false, 3, 1)
@@ -1017,8 +1016,9 @@ MXFA_FWD_F(mxfa_fwd_f64_c_sp_g8, 8, true, false, true)
 MXFA_FWD_F(mxfa_fwd_f64_c_pg_sp_g8, 8, true, true, true)
 // the prefill over a paged cache (causal, as the prefill always is)
 // (the table entry and row address take registers: the 128-query d = 128 form
-// would spill, so paged launches use 64-query work-groups there)
-MXFA_FWD_PG(mxfa_fwd_b64_c_w2_q2_pg, PolBF16<64>, 2, 2)
+// would spill in its loop, so paged launches use 64-query work-groups there;
+// the 128-query d = 64 form spills 9, outside its main loop and twice per masked
+// stage pair)
 MXFA_FWD_PG(mxfa_fwd_b64_c_w3_q2_pg, PolBF16<64>, 3, 2)
 MXFA_FWD_PG(mxfa_fwd_b64_c_w3_q1_pg, PolBF16<64>, 3, 1)
 MXFA_FWD_PG(mxfa_fwd_b128_c_w2_q1_pg, PolBF16<128>, 2, 1)
@@ -1070,16 +1070,14 @@ MXFA_FWD_FEW(mxfa_fwd_b128_few_pg_sp, 128, 4, true, true)
 #undef MXFA_FWD_FEW
 #endif
 
-// The kernel of (policy, causal) compiled for `wps` waves per SIMD with `qt`
-// query tiles per wave (one of the list above); paged: its *_pg form (causal
-// kernels only).
-// bf16 only; fp32 goes through launch_fwd_f32.
+// The kernel of (policy, causal) with `qt` query tiles per wave (one of the list
+// above); paged: its *_pg form (causal kernels only). bf16 only; fp32 goes
+// through launch_fwd_f32.
 template <class Pol, bool CAUSAL>
-static KernelId fwd_kernel_id(int wps, int qt, bool paged) {
+static KernelId fwd_kernel_id(int qt, bool paged) {
     if constexpr (Pol::D == 64) {
-        if (CAUSAL && paged)
-            return qt == 1 ? k_mxfa_fwd_b64_c_w3_q1_pg : wps == 3 ? k_mxfa_fwd_b64_c_w3_q2_pg : k_mxfa_fwd_b64_c_w2_q2_pg;
-        if (CAUSAL) return qt == 1 ? k_mxfa_fwd_b64_c_w3_q1 : wps == 3 ? k_mxfa_fwd_b64_c_w3_q2 : k_mxfa_fwd_b64_c_w2_q2;
+        if (CAUSAL && paged) return qt == 1 ? k_mxfa_fwd_b64_c_w3_q1_pg : k_mxfa_fwd_b64_c_w3_q2_pg;
+        if (CAUSAL) return qt == 1 ? k_mxfa_fwd_b64_c_w3_q1 : k_mxfa_fwd_b64_c_w3_q2;
         return qt == 1 ? k_mxfa_fwd_b64_n_w3_q1 : k_mxfa_fwd_b64_n_w2_q2;
     } else {
         if (CAUSAL && paged) return k_mxfa_fwd_b128_c_w2_q1_pg;
@@ -1091,13 +1089,7 @@ static KernelId fwd_kernel_id(int wps, int qt, bool paged) {
 template <class Pol, bool CAUSAL, int QT>
 static hipError_t launch_fwd_qt(Params p, hipStream_t stream) {
     const dim3 grid(p.B * p.Hq, (p.N + 64 * QT - 1) / (64 * QT));
-    constexpr int kHi = Pol::kWavesFwdCausal;
-    int wps = QT == 1 ? kHi : Pol::kWaves;
-    if constexpr (CAUSAL && kHi > Pol::kWaves && QT > 1) {
-        // enough causal work-groups to fill kHi per CU (256 CUs)
-        if ((long long)grid.x * grid.y >= 256LL * kHi) wps = kHi;
-    }
-    const KernelId id = fwd_kernel_id<Pol, CAUSAL>(wps, QT, p.block_table != nullptr);
+    const KernelId id = fwd_kernel_id<Pol, CAUSAL>(QT, p.block_table != nullptr);
     if (CAUSAL) cu_balance(&p, id, (long long)grid.x * grid.y);
     void *args[] = {&p};
     return launch_kernel(id, grid, dim3(256), args, stream);

@@ -13,11 +13,11 @@
 
 #define MXFA_KERNEL_LIST(X)                                                                   \
     /* forward (fa_fwd.hip): waves per SIMD, 16-query tiles per wave */                      \
-    X(mxfa_fwd_b64_c_w3_q2) X(mxfa_fwd_b64_c_w2_q2) X(mxfa_fwd_b64_c_w3_q1)                   \
+    X(mxfa_fwd_b64_c_w3_q2) X(mxfa_fwd_b64_c_w3_q1)                                           \
     X(mxfa_fwd_b64_n_w2_q2) X(mxfa_fwd_b64_n_w3_q1)                                           \
     X(mxfa_fwd_b128_c_w2_q2) X(mxfa_fwd_b128_c_w2_q1) X(mxfa_fwd_b128_n_w2_q2)                \
     X(mxfa_fwd_f64_c) X(mxfa_fwd_f64_n) X(mxfa_fwd_f64_c_g8) X(mxfa_fwd_f64_n_g8)              \
-    X(mxfa_fwd_b64_c_w2_q2_pg) X(mxfa_fwd_b64_c_w3_q2_pg) X(mxfa_fwd_b64_c_w3_q1_pg)          \
+    X(mxfa_fwd_b64_c_w3_q2_pg) X(mxfa_fwd_b64_c_w3_q1_pg)                                     \
     X(mxfa_fwd_b128_c_w2_q1_pg)                                                               \
     X(mxfa_fwd_f64_c_pg) X(mxfa_fwd_f64_c_pg_g8)                                              \
     X(mxfa_fwd_f64_c_sp_g8) X(mxfa_fwd_f64_c_pg_sp_g8)                                        \

@@ -59,14 +59,13 @@ hipError_t launch_preprocess(const Params &p, int dtype_bf16, int d, hipStream_t
 // delta != 0: the dQ pass computes Delta from p.o_in and writes it to p.delta
 hipError_t launch_bwd_dq(const Params &p, int dtype_bf16, int d, int causal, int delta, hipStream_t stream);
 // p.dkv_ws != nullptr: GQA shapes may split each key block's query heads'
-// stages over several work-groups, with fp32 partials in p.dkv_ws (2 *
-// dkv_split(p, ...) * B * Hkv * N * d floats) and a second, reducing launch
+// stages over several work-groups, with fp32 partials in p.dkv_ws
+// (dkv_workspace_bytes) and a second, reducing launch
 hipError_t launch_bwd_dkv(const Params &p, int dtype_bf16, int d, int causal, hipStream_t stream);
-// partial planes of the split (the most shares of any key block; 1: none)
-int dkv_split(const Params &p, int dtype_bf16, int d, int causal);
-// the workspace the split takes (0: no split): 2 * dkv_split(...) * B * Hkv *
-// N * d floats of partial planes, then 8 bytes per share for the one-launch
-// backward's share flags
+// the workspace the split takes (0: no split): for dK and dV a plane of B * Hkv *
+// N * d floats per share of the key block with the most, then 8 bytes per share
+// for the one-launch backward's share flags. fp32: the planes of a split over
+// 128-key blocks, which the 64-key work-groups keep within
 size_t dkv_workspace_bytes(const Params &p, int dtype_bf16, int d, int causal);
 // The one-launch backward from O (dQ pass with Delta + dK/dV pass, bf16;
 // with p.dkv_ws a GQA split as launch_bwd_dkv, whose reduce runs in the same
