@@ -192,11 +192,13 @@ def test_backward_outside_the_parts():
     assert (dk[:, 77] == 0).all() and (dv[:, 77] == 0).all()
 
 
-@pytest.mark.parametrize("n,nh,nkv,pos0", [(70, 28, 2, 2100), (129, 9, 9, 4000), (256, 32, 4, 1000)])
-def test_chunk_split_over_128_query_blocks(n, nh, nkv, pos0):
+# least: the ranges of 64-query blocks, which a workspace has to hold (0: they take none)
+@pytest.mark.parametrize("n,nh,nkv,pos0,least", [(70, 28, 2, 2100, 10), (129, 9, 9, 4000, 19), (256, 32, 4, 1000, 4),
+                                                 (1200, 14, 2, 1000, 0)])
+def test_chunk_split_over_128_query_blocks(n, nh, nkv, pos0, least):
     """An fp32 chunk whose keys are split over 8-wave work-groups: contiguous and
-    paged alike, with the whole workspace, a smaller one and (where 64-query
-    blocks need none, the last shape) none."""
+    paged alike, with the whole workspace and every smaller one that holds the
+    ranges of 64-query blocks (none where those take none); less is refused."""
     import torch
     import mx230_amd as mx
     rows = -(-(pos0 + n) // 16) * 16
@@ -216,19 +218,20 @@ def test_chunk_split_over_128_query_blocks(n, nh, nkv, pos0):
     tq, tk, tv, tkp, tvp, tt = (torch.from_numpy(x).cuda() for x in (q, k, v, kp, vp, table))
     need = mx.prefill_workspace_bytes(n, pos0, nh, nkv, 64, False)
     one = n * nh * 66 * 4
-    assert need >= 2 * one
-    sizes = [need, need - one + 4] + ([16] if n == 256 else [])
-    for size in sizes:
+    assert need // one > max(least, 1)
+    for size in (need, need - one + 4, least * one if least else 16):
         ws = torch.empty(size, dtype=torch.uint8, device="cuda")
         a, b = (torch.empty(n, nh * 64, device="cuda") for _ in range(2))
-        try:
-            mx.run_prefill_split(tq, tk, tv, a, pos0, nh, nkv, workspace=ws)
-        except mx.MxfaError:  # fewer ranges than 64-query blocks take
-            assert size < need
-            continue
+        mx.run_prefill_split(tq, tk, tv, a, pos0, nh, nkv, workspace=ws)
         mx.run_prefill_paged(tq, tkp, tvp, b, tt, 16, pos0, nh, nkv, split=True, workspace=ws)
         assert torch.equal(a, b)
         assert _close(a.cpu().numpy(), want)
+    if least:
+        ws = torch.empty(least * one - 4, dtype=torch.uint8, device="cuda")
+        with pytest.raises(mx.MxfaError, match="WORKSPACE"):
+            mx.run_prefill_split(tq, tk, tv, a, pos0, nh, nkv, workspace=ws)
+        with pytest.raises(mx.MxfaError, match="WORKSPACE"):
+            mx.run_prefill_paged(tq, tkp, tvp, b, tt, 16, pos0, nh, nkv, split=True, workspace=ws)
 
 
 @pytest.fixture(params=[True, False], ids=["one launch", "two launches"])
@@ -237,6 +240,52 @@ def launches(request):
     old = mx.set_bwd_options(one_launch=request.param)
     yield
     mx.set_bwd_options(**old)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("Hkv", [8, 1], ids=["mha", "gqa"])
+def test_backward_outside_the_parts_everywhere(launches, Hkv, causal):
+    """The rows run again in plain fp32 (a key that no query takes for an infinite
+    element), in one launch and two, with a GQA group's shares, and from a given
+    Delta: the other keys' gradients are those without it."""
+    import torch
+    import mx230_amd as mx
+    rng = np.random.default_rng(10)
+    H, N = 8, 200
+    q, do = (rng.standard_normal((H, N, 64)).astype(np.float32) for _ in range(2))
+    k, v = (rng.standard_normal((Hkv, N, 64)).astype(np.float32) for _ in range(2))
+    q[..., 0] = -np.abs(q[..., 0]) - 0.1
+    k[:, 77, 0] = np.inf
+    keep = np.arange(N) != 77
+    kr, vr = (np.repeat(x, H // Hkv, 0) for x in (k, v))
+    full = [np.zeros((H, N, 64)) for _ in range(3)]
+    for h in range(H):  # one query row at a time over the keys it sees
+        for i in range(N):
+            at = np.flatnonzero(keep[:i + 1] if causal else keep)
+            kk, vv = kr[h, at].astype(np.float64), vr[h, at].astype(np.float64)
+            s = kk @ q[h, i].astype(np.float64) / 8
+            p = np.exp(s - s.max())
+            p /= p.sum()
+            dp = vv @ do[h, i].astype(np.float64)
+            ds = p * (dp - p @ dp)
+            full[0][h, i] = ds @ kk / 8
+            full[1][h, at] += np.outer(ds, q[h, i]) / 8
+            full[2][h, at] += np.outer(p, do[h, i])
+    rq, rk, rv = full[0], *(x.reshape(Hkv, H // Hkv, N, 64).sum(1) for x in full[1:])
+    tq, tk, tv, td = (torch.from_numpy(x[None]).to("cuda") for x in (q, k, v, do))
+    assert (mx.bwd_workspace_bytes(tq, tk, causal) > 0) == (Hkv == 1)
+    o, lse = mx.attention_fwd(tq, tk, tv, causal)
+    given = [torch.empty_like(x) for x in (tq, tk, tv)]
+    delta = torch.empty_like(lse)
+    mx.run_preprocess(td, o, delta)
+    mx.run_bwd_flash(tq, tk, tv, td, lse, delta, *given, causal)
+    for got in (mx.attention_bwd(tq, tk, tv, o, lse, td, causal), given):
+        dq, dk, dv = (x[0].cpu().numpy() for x in got)
+        assert np.abs(dq[..., 1:] - rq[..., 1:]).max() <= 64 * TOL
+        # a key of a GQA group sums its heads' terms
+        assert np.abs(dk[:, keep] - rk[:, keep]).max() <= 64 * TOL * (H // Hkv)
+        assert np.abs(dv[:, keep] - rv[:, keep]).max() <= 64 * TOL * (H // Hkv)
+        assert (dk[:, 77] == 0).all() and (dv[:, 77] == 0).all()
 
 
 @pytest.mark.parametrize("which", ["v", "do"])
