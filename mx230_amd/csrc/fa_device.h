@@ -421,7 +421,10 @@ struct Split3 {
 // us, 500 tokens after 3584 split 48.9 -> 49.5). The later parts of an infinity, or of a value that rounds to one in
 // bf16 (after kPartUp: from 2^104 on), are NaN (inf - inf). Kernels that use
 // parts check their results and, on any that is not finite or a flagged row,
-// run the work-group again in plain fp32 arithmetic.
+// run the work-group again in plain fp32 arithmetic. That takes 10 to 20 times
+// as long (all work-groups of causal B4 H12 N1024: forward 54 -> 775 us, backward
+// 165 -> 1620; the L1 delivers each key's row to 64 rows' lanes), no less with
+// four keys' loads in flight together.
 constexpr float kPartUp = 0x1p24f, kPartDown = 0x1p-24f;
 constexpr float kDsUp = 0x1p48f, kDsDown = 0x1p-48f;
 constexpr float kPartMin = 0x1p-102f;
