@@ -725,21 +725,29 @@ __device__ __forceinline__ void fwd_split_entry(const Params &p) {
     float m = -INFINITY, lsum = 0.f;
 
     // One stage: the online softmax of fwd_stage (FIRST) or, after the
-    // work-group's first stage, fwd_stage_lazy's: scores relative to m, and
-    // m raised only where a lane's sum of p passes kLazySum. A row that precedes
+    // work-group's first stage, fwd_stage_lazy's: m raised only where a lane's sum
+    // of p passes kLazySum. m is subtracted from the finished sums: started at -m,
+    // they are rounded at its size, and not evenly up and down, so the splits of a
+    // long context got weights that were off. kApart: a stage's part of O is summed
+    // from zero and added once, instead of 12 roundings at O's size. Error of O,
+    // relative, rms over 24 draws, with neither, the first, both: one token after
+    // 65535 9.8e-7, 9.1e-7, 3.0e-7 (the fp32 matrix instructions 8.8e-7), after
+    // 4095 3.5e-7, 2.2e-7, 1.9e-7 (4.0e-7). kApart costs 3% of a call and the wide
+    // form's registers (12 to 24 spilled, 49 -> 58 us for 500 tokens after 3584),
+    // where 3.5e-7 against 6.1e-7 is enough without. A row that precedes
     // every key of the first stage (a key split) has m = -inf, and then
     // precedes all later ones too; with finite operands whose first scores all
     // overflow to -inf it does not, and the rows are run again (below).
+    constexpr bool kApart = SPLIT && NW == 4;
     auto compute = [&](auto first, bool edge, int k0) __attribute__((always_inline)) {
         constexpr bool FIRST = decltype(first)::value;
-        const float start = FIRST || m == -INFINITY ? 0.f : -m;
         f32x4 s[2][2];
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
                 Split3 a[1][2];
-                f32x4 c[1][1] = {{f32x4{start, start, start, start}}};
+                f32x4 c[1][1] = {{zero4()}};
                 sm.k.row_frags(a[0], 32 * u + PL::arow(t, l16), g);
                 mma_split_tiles<2, 1, 1>(c, a, qf);
                 s[u][t] = c[0][0];
@@ -758,6 +766,7 @@ __device__ __forceinline__ void fwd_split_entry(const Params &p) {
                 }
             }
         }
+        const float base = m == -INFINITY ? 0.f : m;  // what p is relative to
         f32x4 pv[2][2];
         auto exps = [&](float sub) __attribute__((always_inline)) {
             float ls = 0.f;
@@ -785,34 +794,48 @@ __device__ __forceinline__ void fwd_split_entry(const Params &p) {
                     for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[u][t][r]);
                 }
             }
-            mx = xg_max(mx);  // relative to m after the first stage
-            const float shift = FIRST ? (mx == -INFINITY ? 0.f : mx) : fmaxf(mx, 0.f);
-            m = FIRST ? mx : m + shift;
+            mx = fmaxf(xg_max(mx), m);
+            const float to = mx == -INFINITY ? 0.f : mx;
             if constexpr (!FIRST) {
-                const float corr = fast_exp2(-shift);
+                const float corr = fast_exp2(base - to);
                 lsum *= corr;
 #pragma unroll
                 for (int xt = 0; xt < XT; ++xt) acc[xt] *= corr;
             }
-            lsum += exps(shift);
+            m = mx;
+            lsum += exps(to);
         };
         if constexpr (FIRST) {
             raise();
         } else {
-            const float ls = exps(0.f);
+            const float ls = exps(base);
             if (__builtin_amdgcn_ballot_w64(ls > kLazySum) != 0) {
                 raise();
             } else {
                 lsum += ls;
             }
         }
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const Split3 pf[1] = {split3(pv[u][0], pv[u][1])};
+        if constexpr (kApart) {
+            const Split3 pf[2][1] = {{split3(pv[0][0], pv[0][1])}, {split3(pv[1][0], pv[1][1])}};
 #pragma unroll
             for (int xt = 0; xt < XT; ++xt) {
-                const Split3 a[1] = {sm.v.chain_a(16 * xt, 32 * u, g, l16)};
-                acc[xt] = mma_split<1>(a, pf, acc[xt]);
+                f32x4 c = zero4();
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const Split3 a[1] = {sm.v.chain_a(16 * xt, 32 * u, g, l16)};
+                    c = mma_split<1>(a, pf[u], c);
+                }
+                acc[xt] += c;
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const Split3 pf[1] = {split3(pv[u][0], pv[u][1])};
+#pragma unroll
+                for (int xt = 0; xt < XT; ++xt) {
+                    const Split3 a[1] = {sm.v.chain_a(16 * xt, 32 * u, g, l16)};
+                    acc[xt] = mma_split<1>(a, pf, acc[xt]);
+                }
             }
         }
     };
