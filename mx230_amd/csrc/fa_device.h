@@ -417,8 +417,9 @@ struct Split3 {
 // flagged, split_row), those of dP by kPartUp too, which keeps dS (scaled
 // kDsUp then) in range as well, and the sums at the end. Without it V or dO of
 // size 2^-115 gave dQ and dK errors of 9e-6 and of 2^-120, 2.9e-4, instead of
-// 3e-7. It costs 1.3% (causal B4 H12 N1024 forward and backward 185.6 -> 188.0
-// us, 500 tokens after 3584 split 48.9 -> 49.5). The later parts of an infinity, or of a value that rounds to one in
+// 3e-7. It costs 1 to 4% (us, forward + backward without and with: causal B4 H12
+// N1024 192 -> 195, B1 H12 N4096 650 -> 666, non-causal B6 16/8 heads of 75 rows
+// 28.4 -> 29.5). The later parts of an infinity, or of a value that rounds to one in
 // bf16 (after kPartUp: from 2^104 on), are NaN (inf - inf). Kernels that use
 // parts check their results and, on any that is not finite or a flagged row,
 // run the work-group again in plain fp32 arithmetic. That takes 10 to 20 times
@@ -923,6 +924,8 @@ constexpr int tile_loads() {
 // A row's two 8-element operands of a lane (k-steps 0 and 1), times mul, as
 // parts; zeros for rows that are not there. True for the whole wave if all of
 // some row's values are below kPartMin and not all 0: its parts are not 24 bits.
+// (Rows are combined on the scalar unit: by cross-lane maxima causal B1 6/3 heads of
+// 1060 rows took 40.9 + 56.0 us, forward and backward, instead of 39.7 + 54.2.)
 __device__ __forceinline__ bool split_row(Split3 (&f)[2], const float *row, int g, float mul, bool valid) {
     float mx = 0.f;
 #pragma unroll
@@ -935,8 +938,10 @@ __device__ __forceinline__ bool split_row(Split3 (&f)[2], const float *row, int 
         for (int e = 0; e < 4; ++e) mx = fmaxf(mx, fmaxf(fabsf(a[e]), fabsf(b[e])));
         f[kc] = split3(a, b);
     }
-    mx = xg_max(mx);
-    return __builtin_amdgcn_ballot_w64(mx > 0.f && mx < kPartMin) != 0;
+    uint64_t some = __builtin_amdgcn_ballot_w64(mx > 0.f), enough = __builtin_amdgcn_ballot_w64(mx >= kPartMin);
+    some |= some >> 32;  // a row's four lanes are 16 apart
+    enough |= enough >> 32;
+    return (((some | some >> 16) & ~(enough | enough >> 16)) & 0xffff) != 0;
 }
 
 // True for every wave of the work-group if any of its lanes holds a value that
