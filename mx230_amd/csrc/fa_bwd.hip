@@ -1121,7 +1121,7 @@ __device__ __forceinline__ void bwd_fused_entry(const Params &p) {
 // waves, 64 rows per work-group (16 per wave, in registers as parts), 64 rows
 // of the other side per stage. Those pass through registers, loaded one stage
 // ahead, and are split once per work-group into one 48 KB LDS buffer. The dQ
-// pass holds three work-groups per CU (156 VGPRs), the dK/dV pass two (252),
+// pass holds three work-groups per CU (156 VGPRs), the dK/dV pass two (248),
 // whose splitting, softmax and matrix products overlap.
 //
 // Bound: the matrix unit and what of the splitting it does not hide. A wave's

@@ -604,9 +604,9 @@ __device__ __forceinline__ void fwd_few_entry(const Params &p) {
 // instructions, over half of them the splitting. Event medians on one card,
 // us, against v_mfma_f32_16x16x4_f32 on the same tiles: causal B4 H12 N1024
 // 79.5 -> 54, B4 H12 N4096 806 -> 523 (197 TFLOP/s), non-causal B1 H12 N4096
-// 411 -> 318, B1 H1 N256 16.0 -> 14.1. Error of O against 64 bits, same
-// shapes: 3.5e-7 -> 3.0e-7, 5.1e-7 -> 4.5e-7, 1.2e-6 -> 1.1e-6, 4.4e-7 ->
-// 4.1e-7. Two 16-query tiles per wave, the waves in pairs over half a stage's
+// 411 -> 318, B1 H1 N256 16.0 -> 14.1. Error of O against 64 bits: causal
+// N1000 3.4e-7 -> 2.1e-7, N4096 5.1e-7 -> 3.8e-7, non-causal N4096 1.2e-6 ->
+// 1.0e-6, N256 4.4e-7 -> 2.6e-7. Two 16-query tiles per wave, the waves in pairs over half a stage's
 // keys each (half the LDS reads) ran 54.6, 570, 338 and 14.6: 250 VGPRs leave
 // two waves per SIMD.
 struct FwdSplitSmem {
